@@ -52,6 +52,9 @@ KERNEL_FIELDS = {
     "k_ac_mu_ww": 3,        # dvdxi ww1 -> ww
     "k_ac_theta": 11,       # t t_tend t_save u v ww ww_m ww1 -> t t_2save ww_m
     "k_ac_wsolve": 19,      # t_2save c2a alt rw_tend cqw w ph ph_tend ph_save phb ww t t_save pm1 -> w ph al p pm1
+    # u v u_save v_save ru_m rv_m ww1 ww_m t t_tend t_save w ph ph_tend ph_save phb c2a alt rw_tend
+    # cqw pm1 -> ru_m rv_m ww_m t w ph al p pm1
+    "k_ac_column": 30,
     "k_small_finish": 19,   # 5x*_2 5x*_save ww ww1 h_diabatic -> 5x*_2 ww
     "k_adv_scalar": 5,      # q ru_m rv_m ww_m -> advect_tend
     "k_update_scalar": 5,   # advect_tend q_tend q q_old -> q

@@ -21,6 +21,8 @@
 #define __shared__ static
 #define WRFMI_GLOBAL_AS
 #define WRFMI_CONST_AS
+// dynamic LDS: one block at a time runs, so one buffer of a CU's LDS serves every launch
+#define WRFMI_DYN_LDS(name) alignas(16) static char name[160 * 1024]
 
 struct dim3 {
   unsigned x, y, z;

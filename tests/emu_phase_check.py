@@ -74,6 +74,16 @@ CASES = {
                          lbc=52),
     "spec_mixed": dict(nx=17, ny=12, nz=10, bc="specified", n_passive=2, n_bubbles=1, seed=43, lbc=53, pd=(1, 1),
                        opts=dict(have_bcs_scalar=1, diff_6th_opt=2, damp_opt=3, zdamp=5000.0)),
+    # k_ac_column's tiles: a last tile of one column, a single tile, levels at and past what
+    # each tile shape holds (48, 64, 80 on 32 columns; 96 on 16; 192 on 8), and columns too
+    # tall for any tile (the routine kernels)
+    "col_33": dict(nx=33, ny=7, nz=49, bc="periodic", n_bubbles=1, seed=61),
+    "col_28": dict(nx=28, ny=8, nz=65, bc="open", n_bubbles=1, seed=62),
+    "col_64": dict(nx=64, ny=7, nz=81, bc="periodic", n_bubbles=1, seed=63, pad_i=1),
+    "col_spec": dict(nx=33, ny=9, nz=48, bc="specified", n_bubbles=1, seed=64, lbc=54),
+    "col_16": dict(nx=17, ny=7, nz=97, bc="periodic", n_bubbles=1, seed=65),
+    "col_8": dict(nx=9, ny=7, nz=193, bc="periodic", n_bubbles=1, seed=66),
+    "col_tall": dict(nx=9, ny=7, nz=321, bc="open", n_bubbles=1, seed=67),
     "pd_mixed_unaligned": dict(nx=14, ny=11, nz=8, bc_x="open", bc_y="periodic", n_passive=1, n_bubbles=1, seed=28,
                                pad_i=1, pd=(0, 1)),
 }

@@ -42,6 +42,17 @@ def test_emulated_kernels_match_oracle(emu_env, case, order, nsteps):
     assert "OK" in r.stdout
 
 
+@pytest.mark.parametrize("case,order", [("col_33", 0), ("col_28", 1), ("col_64", 0), ("col_spec", 1), ("col_16", 0),
+                                        ("col_8", 1), ("col_tall", 0)])
+def test_emulated_column_tiles_match_oracle(emu_env, case, order):
+    """The acoustic column kernel at the edges of its tile shapes, and the routine kernels
+    beyond them, bit for bit with the oracle."""
+    r = subprocess.run([sys.executable, os.path.join(HERE, "emu_phase_check.py"), case, str(order), "1"],
+                       env=emu_env, capture_output=True, text=True, timeout=900)
+    assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-4000:]
+    assert "OK" in r.stdout
+
+
 def test_emulated_host_array_registry(emu_env):
     r = subprocess.run([sys.executable, os.path.join(HERE, "emu_phase_check.py"), "registry"],
                        env=emu_env, capture_output=True, text=True, timeout=300)

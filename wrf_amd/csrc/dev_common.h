@@ -78,6 +78,11 @@ struct CPtr {
   HDI T operator[](int i) const { return ((const WRFMI_CONST_AS T *)p)[i]; }
 };
 
+// Dynamic LDS of a workgroup, sized at the launch
+#ifndef WRFMI_DYN_LDS
+#define WRFMI_DYN_LDS(name) extern __shared__ __attribute__((aligned(16))) char name[]
+#endif
+
 // Device view of wrfmi_state: same layout, arrays as FPtr (1-D level arrays as CPtr)
 struct DState {
 #define WRFMI_DPTR(n) FPtr<float> n;
@@ -118,7 +123,10 @@ struct KArgs {
   unsigned long long qt_stride;  // one grid field (elements) apart
   int tnx, tny, tnz;  // tiles of the current launch in i, j and k (see tile3)
   int routine;        // Routine: R_FUSED in the whole step and the grouped entry points
+  int keep;           // k_ac_column: the column work it stores for its callers (kKeep*)
 };
+constexpr int kKeepWW = 1;   // omega (small_step_finish reads it after the last substep)
+constexpr int kKeepAux = 2;  // t_2save and gamma (state fields no later kernel of a step reads)
 
 // One field of a batched halo fill (set_physical_bc3d/2d on up to 16 fields per launch)
 struct HaloField {

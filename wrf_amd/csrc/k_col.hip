@@ -1,0 +1,688 @@
+// The column part of one acoustic substep in one kernel: advance_mu_t
+// (module_small_step_em.F:969-1175), advance_w (1178-1469), sumflux (1473-1633) and
+// calc_p_rho (438-568) for the columns of a tile.
+//
+// Everything after advance_uv is local to a column, given u, v and t_save of its
+// neighbours, so a workgroup takes a tile of C columns of one row through the whole
+// substep: C lanes along i times blockDim.y level lanes of up to TASKS levels each, every
+// level of the tile in flight at once.  Only the four recurrences in k (the mass-divergence
+// sum, the omega scan, the tridiagonal forward and back sweeps) run serially, one lane per
+// column, and those read and write LDS; every division that does not depend on a recurrence
+// is formed by the level lanes beforehand.  The expressions and their order are those of
+// the routine kernels in k_small.hip (k_ac_div, k_ac_mu_ww, k_ac_theta, k_ac_wsolve), which
+// keep the forms with the reference's argument lists and the columns too tall for LDS.
+//
+// What bounds it: on large domains the tile's reads and writes, 31 fields per mass point
+// against the 42 of the four routine kernels; the workgroups that LDS and registers let onto
+// a CU (three of a 32-column, 80-level tile) have to hide each other's serial stretches and
+// barriers.  On small ones the serial sweeps: a lane alone issues one dependent instruction
+// after another, so their loops hold little else (see sweep_up).
+//
+// Task m of a column is mass level k = m + 1 and w level kw = m + 2.  LDS arrays, one value
+// per task and column:
+//   W  dnw*dvdxi, then the omega increments, then omega      A  c2a*alt*t_2ave
+//   B  the pressure term    G  the column values             R  rhs, then the final ph
+// and, over W, A, B and G, the tridiagonal rows Q, then gamma and w in their place.
+#include "kernels.h"
+
+namespace wrfmi {
+
+struct alignas(16) L4 {  // four coefficients of one level
+  float x, y, z, w;
+};
+// a row of the tridiagonal system: sub-, main and super-diagonal, right-hand side
+template <typename CT>
+struct alignas(16) Row {
+  CT a, b, c, w;
+};
+
+// The launch's arguments, to be read again by every phase of the kernel: the pointers of all
+// phases together are more than the scalar registers hold, and the compiler would park them
+// in vector lanes (a readlane per use) instead of loading them again.
+DEVI const KArgs *karg_ptr(const KArgs &a) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return (const KArgs *)(const WRFMI_CONST_AS KArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+#else
+  return &a;
+#endif
+}
+DEVI const KArgs *karg_ptr(const BatchArgs &b) {
+  return (const KArgs *)(b.m + b.lut[xcd_logical(blockIdx.x, b.total)]);
+}
+DEVI const KArgs &again(const KArgs *p) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const WRFMI_CONST_AS KArgs *q = (const WRFMI_CONST_AS KArgs *)p;
+  asm volatile("" : "+s"(q));
+  return *(const KArgs *)q;
+#else
+  return *p;
+#endif
+}
+#define WRFMI_PHASE \
+  const KArgs &a = again(pa); \
+  const Dm &d = a.d; \
+  const DState &s = dstate(a); \
+  (void)d
+
+// sumflux of ru_m and rv_m in the column (x, j) outside the mass points (x = ide or
+// j = jde): levels 1 + n, 1 + n + step, ...
+DEVI void sumflux_edge(const KArgs &a, int x, int j, int n, int step) {
+  const Dm &d = a.d;
+  const DState &s = dstate(a);
+  const bool mi = x <= d.ide - 1, mj = j <= d.jde - 1, first = a.iteration == 1, last = a.iteration == a.nsmall;
+  const float nsf = (float)a.nsmall;
+  const Off q2 = X2(d, x, j);
+  for (int k = 1 + n; k <= d.kde; k += step) {
+    const Off o = X3(d, x, k, j);
+    if (k < d.kde) {
+      float rum = first ? 0.f : s.ru_m[o], rvm = first ? 0.f : s.rv_m[o];
+      if (mj) rum = rum + s.u_2[o];
+      if (mi) rvm = rvm + s.v_2[o];
+      if (last) {
+        if (mj) rum = rum / nsf + (s.c1h[X1(d, k)] * s.muu[q2] + s.c2h[X1(d, k)]) * s.u_save[o] / s.msfuy[q2];
+        if (mi) rvm = rvm / nsf + (s.c1h[X1(d, k)] * s.muv[q2] + s.c2h[X1(d, k)]) * s.v_save[o] * s.msfvx_inv[q2];
+      }
+      s.ru_m[o] = rum;
+      s.rv_m[o] = rvm;
+    } else if (first) {
+      s.ru_m[o] = 0.f;
+      s.rv_m[o] = 0.f;
+    }
+    if (first) s.ww_m[o] = 0.f;
+  }
+}
+
+// A recurrence over m = 0 .. n-1 on one lane: body(m, vals) in order, vals[f] = load(f, m)
+// read from LDS a block of levels ahead (the loads must not read what the body writes at a
+// later m).
+template <int NF, typename T, typename Load, typename Body>
+DEVI void serial_up(int n, Load &&load, Body &&body) {
+  constexpr int BL = sizeof(T) * NF <= 4 ? 8 : 4;
+  T cur[BL][NF], nxt[BL][NF];
+#pragma unroll
+  for (int r = 0; r < BL; r++)
+#pragma unroll
+    for (int f = 0; f < NF; f++) cur[r][f] = load(f, imin(r, n - 1));
+  int mb = 0;
+  for (; mb + BL <= n; mb += BL) {
+#pragma unroll
+    for (int r = 0; r < BL; r++)
+#pragma unroll
+      for (int f = 0; f < NF; f++) nxt[r][f] = load(f, imin(mb + BL + r, n - 1));
+#pragma unroll
+    for (int r = 0; r < BL; r++) body(mb + r, cur[r]);
+#pragma unroll
+    for (int r = 0; r < BL; r++)
+#pragma unroll
+      for (int f = 0; f < NF; f++) cur[r][f] = nxt[r][f];
+  }
+#pragma unroll
+  for (int r = 0; r < BL - 1; r++)
+    if (mb + r < n) body(mb + r, cur[r]);
+}
+
+// The forward elimination of one column (rows C apart), one row per level: gamma goes to .c
+// and the forward value to .w.  A lane runs it alone, so its time is the count of dependent
+// instructions.  In float the IEEE reciprocal 1/(b - a gam) is formed without the division's
+// scaling steps: for |x| in [2^-100, 2^100] the hardware reciprocal (within 1 ulp) and two
+// residual corrections give the correctly rounded value (checked for every significand).  A
+// block with a pivot outside that range is done again with the division.  Against the
+// division in the loop, each array loaded by its own instruction: 14.7 against 8.6 thousand
+// cycles for 40 levels.
+template <typename CT, int C>
+DEVI void sweep_up(Row<CT> *q, int n, CT &gam, CT &wfe) {
+  constexpr int BL = sizeof(CT) == 4 ? 4 : 2;
+  Row<CT> cur[BL];
+#pragma unroll
+  for (int r = 0; r < BL; r++) cur[r] = q[imin(r, n - 1) * C];
+  auto level = [&](const Row<CT> &y, CT alpha, CT &g, CT &w) {
+    g = y.c * alpha;
+    w = (y.w - y.a * w) * alpha;
+  };
+  auto store = [&](int m, CT g, CT w) {
+    // the double form keeps the forward value as the sum of two floats
+    if (sizeof(CT) == 8 && m < n - 1) w = (CT)(float)w + (CT)(float)((double)w - (double)(float)w);
+    q[m * C].c = g;
+    q[m * C].w = w;
+  };
+  int mb = 0;
+  for (; mb + BL <= n; mb += BL) {
+    Row<CT> nxt[BL];
+#pragma unroll
+    for (int r = 0; r < BL; r++) nxt[r] = q[imin(mb + BL + r, n - 1) * C];
+    CT g[BL], w[BL];
+    CT g1 = gam, w1 = wfe;
+    bool divide = true;
+#ifdef __HIP_DEVICE_COMPILE__
+    if constexpr (sizeof(CT) == 4) {
+      float lo = 1.f, hi = 1.f;
+#pragma unroll
+      for (int r = 0; r < BL; r++) {
+        const float x = cur[r].b - cur[r].a * g1;
+        lo = fminf(lo, fabsf(x));
+        hi = fmaxf(hi, fabsf(x));
+        float al = __builtin_amdgcn_rcpf(x);
+        al = fmaf(fmaf(-x, al, 1.f), al, al);
+        al = fmaf(fmaf(-x, al, 1.f), al, al);
+        level(cur[r], al, g1, w1);
+        g[r] = g1;
+        w[r] = w1;
+      }
+      divide = !(lo >= 0x1p-100f && hi <= 0x1p100f);
+    }
+#endif
+    if (divide) {
+      g1 = gam;
+      w1 = wfe;
+#pragma unroll
+      for (int r = 0; r < BL; r++) {
+        level(cur[r], CT(1) / (cur[r].b - cur[r].a * g1), g1, w1);
+        g[r] = g1;
+        w[r] = w1;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < BL; r++) store(mb + r, g[r], w[r]);
+    gam = g1;
+    wfe = w1;
+#pragma unroll
+    for (int r = 0; r < BL; r++) cur[r] = nxt[r];
+  }
+#pragma unroll
+  for (int r = 0; r < BL - 1; r++)
+    if (mb + r < n) {
+      level(cur[r], CT(1) / (cur[r].b - cur[r].a * gam), gam, wfe);
+      store(mb + r, gam, wfe);
+    }
+}
+
+template <typename ARGS, typename CT, bool COMP, int C, int TASKS>
+__global__ void __launch_bounds__(kColThreads, sizeof(CT) == 4 ? 6 : 4) k_ac_column(ARGS args) {
+  const KArgs *const pa = karg_ptr(args);
+  Tile3 T;
+  (void)kargs(args, T);
+  const int KL = (int)blockDim.y, kl = (int)threadIdx.y, col = (int)threadIdx.x;
+  int ia, j, nz, ni, sj, alo, ahi, ids, ide;
+  Off ob, o2;  // level k of the lane's column at ob + k*ni
+  {
+    WRFMI_PHASE;
+    (void)s;
+    ia = col_tile_ia(d, C) + T.bx * C;
+    j = d.jds + T.by;
+    nz = d.kde - 1;
+    ni = d.ni;
+    sj = d.sj;
+    ids = d.ids;
+    ide = d.ide;
+    // the points outside the mass points (row jde, column ide) take sumflux only
+    if (j == d.jde) {
+      const int x = ia + col;
+      if (x >= ids && x < ide) sumflux_edge(a, x, j, kl, KL);
+    }
+    if (ia + C >= ide) sumflux_edge(a, ide, j, kl * C + col, KL * C);
+    if (j == d.jde) return;
+    // columns that advance, alo..ahi: a specified domain's outermost ones are the boundary kernels'
+    const bool spec = a.c.specified || a.c.nested, sx = spec && !a.c.periodic_x;
+    alo = sx ? ids + 1 : ids;
+    ahi = sx ? ide - 2 : ide - 1;
+    if (spec && (j == d.jds || j == d.jde - 1)) ahi = alo - 1;
+    ob = X3(d, ia + col, 0, j);
+    o2 = X2(d, ia + col, j);
+  }
+  const int i = ia + col;
+  const bool in = i >= ids && i <= ide - 1, act = i >= alo && i <= ahi, serial = act && kl == 0;
+  WRFMI_DYN_LDS(lds);
+  float *const W = (float *)lds, *const A = W + C * nz, *const B = A + C * nz, *const G = B + C * nz;
+  Row<CT> *const Q = (Row<CT> *)lds;
+  float *const R = (float *)(Q + C * nz);
+  L4 *const LA = (L4 *)(R + C * nz), *const LB = LA + nz;  // level k at [k - 1]: c1h c2h rdnw dnw, c1f c2f fnm fnp
+  float *const c_dmdt = G, *const c_mu = c_dmdt + C, *const c_muts = c_mu + C, *const c_muave = c_muts + C;
+
+  // the serial lanes' column values, loaded ahead of their turns
+  float wsfc = 0.f, s_mu = 0.f, s_mut = 0.f, s_mu_tend = 0.f, s_ww = 0.f, s_ww1 = 0.f;
+  float msfty = 1.f, mut = 1.f;
+  {
+    WRFMI_PHASE;
+    for (int k = 1 + kl * C + col; k <= nz; k += KL * C) {
+      LA[k - 1] = L4{s.c1h[X1(d, k)], s.c2h[X1(d, k)], s.rdnw[X1(d, k)], s.dnw[X1(d, k)]};
+      LB[k - 1] = L4{s.c1f[X1(d, k)], s.c2f[X1(d, k)], s.fnm[X1(d, k)], s.fnp[X1(d, k)]};
+    }
+    if (in) {
+      msfty = s.msfty[o2];
+      mut = s.mut[o2];
+    }
+    if (serial) {
+      const Off l1 = ob + ni, l2 = l1 + ni, l3 = l2 + ni;
+      s_mu = s.mu_2[o2];
+      s_mut = mut;
+      s_mu_tend = s.mu_tend[o2];
+      s_ww = s.ww[l1];
+      s_ww1 = s.ww1[l1];
+      // advance_w's lower boundary (1383-1395): w(1) from u, v extrapolated to the surface by
+      // cf1..cf3 and the terrain slopes on both sides of the point
+      const FPtr<float> u = s.u_2, v = s.v_2, ht = s.ht;
+      const float cf1 = s.cf1, cf2 = s.cf2, cf3 = s.cf3;
+      wsfc = msfty * .5f * s.rdy *
+                 ((ht[o2 + ni] - ht[o2]) * (cf1 * v[l1 + sj] + cf2 * v[l2 + sj] + cf3 * v[l3 + sj]) +
+                  (ht[o2] - ht[o2 - ni]) * (cf1 * v[l1] + cf2 * v[l2] + cf3 * v[l3])) +
+             s.msftx[o2] * .5f * s.rdx *
+                 ((ht[o2 + 1] - ht[o2]) * (cf1 * u[l1 + 1] + cf2 * u[l2 + 1] + cf3 * u[l3 + 1]) +
+                  (ht[o2] - ht[o2 - 1]) * (cf1 * u[l1] + cf2 * u[l2] + cf3 * u[l3]));
+      s.w_2[l1] = wsfc;
+    }
+  }
+  __syncthreads();
+
+  // ---- dvdxi and sumflux of the horizontal fluxes.  In each phase every task's loads come
+  // before the first task's stores, which would hold them back.
+  float q_dv[TASKS];
+  if (in) {
+    WRFMI_PHASE;
+    const bool first = a.iteration == 1, last = a.iteration == a.nsmall;
+    const float nsf = (float)a.nsmall, rdx = s.rdx, rdy = s.rdy;
+    const float muu0 = s.muu[o2], muu1 = s.muu[o2 + 1], muv0 = s.muv[o2], muv1 = s.muv[o2 + ni], msftx = s.msftx[o2];
+    const float msfuy0 = s.msfuy[o2], msfuy1 = s.msfuy[o2 + 1], mvi0 = s.msfvx_inv[o2], mvi1 = s.msfvx_inv[o2 + ni];
+    float u0[TASKS], u1[TASKS], v0[TASKS], v1[TASKS], us0[TASKS], us1[TASKS], vs0[TASKS], vs1[TASKS];
+    float rum[TASKS], rvm[TASKS];
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const Off o = ob + imin(kl + t * KL + 1, nz) * ni;
+      u0[t] = s.u_2[o];
+      u1[t] = s.u_2[o + 1];
+      v0[t] = s.v_2[o];
+      v1[t] = s.v_2[o + sj];
+      us0[t] = s.u_save[o];
+      us1[t] = s.u_save[o + 1];
+      vs0[t] = s.v_save[o];
+      vs1[t] = s.v_save[o + sj];
+    }
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const Off o = ob + imin(kl + t * KL + 1, nz) * ni;
+      rum[t] = rvm[t] = 0.f;
+      if (!first) {
+        rum[t] = s.ru_m[o];
+        rvm[t] = s.rv_m[o];
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const int m = kl + t * KL;
+      if (m < nz) {
+        const Off o = ob + (m + 1) * ni;
+        const L4 la = LA[m];
+        // the large-step fluxes at both faces (x/1 is x: no division on a Cartesian domain)
+        float U0 = (la.x * muu0 + la.y) * us0[t], U1 = (la.x * muu1 + la.y) * us1[t];
+        if (msfuy0 != 1.f) U0 = U0 / msfuy0;
+        if (msfuy1 != 1.f) U1 = U1 / msfuy1;
+        const float V0 = (la.x * muv0 + la.y) * vs0[t] * mvi0, V1 = (la.x * muv1 + la.y) * vs1[t] * mvi1;
+        float ru = rum[t] + u0[t], rv = rvm[t] + v0[t];
+        if (last) {
+          ru = ru / nsf + U0;
+          rv = rv / nsf + V0;
+        }
+        s.ru_m[o] = ru;
+        s.rv_m[o] = rv;
+        q_dv[t] = msftx * msfty * (rdy * ((v1[t] + V1) - (v0[t] + V0)) + rdx * ((u1[t] + U1) - (u0[t] + U0)));
+        W[m * C + col] = la.w * q_dv[t];
+      }
+    }
+    if (first && kl == 0) {
+      s.ru_m[ob + (nz + 1) * ni] = 0.f;
+      s.rv_m[ob + (nz + 1) * ni] = 0.f;
+    }
+  }
+  // the next phases' own-level inputs: on their way while the column integral and the omega
+  // scan run
+  float q_t[TASKS], q_tt[TASKS], q_t1[TASKS], q_alt[TASKS], q_c2a[TASKS], q_w1[TASKS], q_wwm[TASKS];
+  if (in) {
+    WRFMI_PHASE;
+    const bool first = a.iteration == 1;
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const Off o = ob + imin(kl + t * KL + 2, nz + 1) * ni;
+      q_w1[t] = s.ww1[o];
+      q_wwm[t] = 0.f;
+      if (!first) q_wwm[t] = s.ww_m[o];
+    }
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const Off o = ob + imin(kl + t * KL + 1, nz) * ni;
+      q_t[t] = s.t_2[o];
+      q_tt[t] = s.t_tend[o];
+      q_t1[t] = s.t_save[o];
+      q_alt[t] = s.alt[o];
+      q_c2a[t] = s.c2a[o];
+    }
+  }
+  __syncthreads();
+
+  // ---- the column integral and the mass update
+  if (serial) {
+    WRFMI_PHASE;
+    const float dts = a.dts, epssm = a.c.epssm;
+    float dmdt = 0.f, comp = 0.f;
+    serial_up<1, float>(nz, [&](int, int m) { return W[m * C + col]; }, [&](int, const float *y) {
+      if (COMP) two_sum_acc(dmdt, comp, y[0]);
+      else dmdt = dmdt + y[0];
+    });
+    if (COMP) dmdt = dmdt + comp;
+    float mu = s_mu;
+    float muave = mu;
+    mu = mu + dts * (dmdt + s_mu_tend);
+    s.mu_2[o2] = mu;
+    s.mudf[o2] = (dmdt + s_mu_tend);
+    const float muts = s_mut + mu;
+    s.muts[o2] = muts;
+    muave = .5f * ((1.f + epssm) * mu + (1.f - epssm) * muave);
+    s.muave[o2] = muave;
+    c_dmdt[col] = dmdt;
+    c_mu[col] = mu;
+    c_muts[col] = muts;
+    c_muave[col] = muave;
+  }
+  __syncthreads();
+  float mu = 0.f, muts = 1.f, muave = 0.f;
+  if (act) {
+    WRFMI_PHASE;
+    const float dmdt = c_dmdt[col], mu_tend = s.mu_tend[o2];
+    mu = c_mu[col];
+    muts = c_muts[col];
+    muave = c_muave[col];
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const int m = kl + t * KL;
+      if (m < nz - 1) {
+        const L4 la = LA[m];
+        float y = la.w * ((la.x * dmdt) + q_dv[t] + (la.x * mu_tend));
+        if (msfty != 1.f) y = y / msfty;
+        W[m * C + col] = y;
+      }
+    }
+  }
+  __syncthreads();
+  // ---- the omega scan: W(m) becomes omega at w level m + 2 before ww1 is taken off
+  if (serial) {
+    WRFMI_PHASE;
+    float prev = s_ww;
+    s.ww[ob + ni] = prev - s_ww1;
+    serial_up<1, float>(nz - 1, [&](int, int m) { return W[m * C + col]; }, [&](int m, const float *y) {
+      prev = prev - y[0];
+      W[m * C + col] = prev;
+    });
+  }
+  __syncthreads();
+  float ww_bot = 0.f;  // omega at the surface (on the lowest level's lanes)
+  if (in) {
+    WRFMI_PHASE;
+    const bool first = a.iteration == 1, last = a.iteration == a.nsmall, keep_ww = a.keep & kKeepWW;
+    const float nsf = (float)a.nsmall;
+    // sumflux of omega at a w level
+    auto sum_ww = [&](Off o, float wwm, float ww, float w1) {
+      wwm = wwm + ww;
+      if (last) wwm = wwm / nsf + w1;
+      s.ww_m[o] = wwm;
+    };
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const int m = kl + t * KL;
+      if (m < nz) {
+        const Off o = ob + (m + 2) * ni;
+        float ww = W[m * C + col] - q_w1[t];
+        // the lid, and a specified domain's outermost columns: as they are
+        if (m == nz - 1 || !act) ww = s.ww[o];
+        else if (keep_ww) s.ww[o] = ww;
+        sum_ww(o, q_wwm[t], ww, q_w1[t]);
+        W[m * C + col] = ww;
+      }
+    }
+    if (kl == 0) {
+      ww_bot = s.ww[ob + ni];
+      sum_ww(ob + ni, first ? 0.f : s.ww_m[ob + ni], ww_bot, s.ww1[ob + ni]);
+    }
+  }
+  __syncthreads();
+
+  // ---- theta, t_2ave; rhs of the w equation (1324-1371); what calc_p_rho takes from them
+  float pX[TASKS], pY[TASKS];
+  float P_lid = 0.f;  // the lid equation's product, in its own order
+  if (act) {
+    WRFMI_PHASE;
+    const wrfmi_config &c = a.c;
+    const bool z2 = c.phi_adv_z == 2, keep_aux = a.keep & kKeepAux;
+    const float dts = a.dts, epssm = c.epssm, rdx = s.rdx, rdy = s.rdy;
+    const float c1f_top = s.c1f[X1(d, nz + 1)], c2f_top = s.c2f[X1(d, nz + 1)];
+    const float msftx = s.msftx[o2];
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const int m = kl + t * KL, k = m + 1;
+      if (m < nz) {
+        const bool top = m == nz - 1;
+        const Off o = ob + k * ni;
+        const L4 la = LA[m], lb = LB[m], lbp = LB[top ? m : m + 1];
+        const float c2a = q_c2a[t], alt = q_alt[t], t1 = q_t1[t], tv = q_t[t];
+        const float t1p = s.t_save[o + ni], t1m = s.t_save[k >= 2 ? o - ni : o];
+        const float ww_hi = W[m * C + col], ww_lo = m == 0 ? ww_bot : W[(m - 1) * C + col];
+        float th = tv + msfty * dts * q_tt[t];
+        const float wdtn_hi = !top ? ww_hi * (lbp.z * t1p + lbp.w * t1) : 0.f;
+        const float wdtn_lo = (k >= 2) ? ww_lo * (lb.z * t1 + lb.w * t1m) : 0.f;
+        th = th - dts * msfty *
+                      (msftx * (.5f * rdy * (s.v_2[o + sj] * (s.t_save[o + sj] + t1) - s.v_2[o] * (t1 + s.t_save[o - sj])) +
+                                .5f * rdx * (s.u_2[o + 1] * (s.t_save[o + 1] + t1) - s.u_2[o] * (t1 + s.t_save[o - 1]))) +
+                       la.z * (wdtn_hi - wdtn_lo));
+        const float D = (la.x * muts + la.y) * (K_T0 + t1);
+        float v1 = .5f * ((1.f + epssm) * th + (1.f - epssm) * tv);
+        v1 = (v1 + (la.x * muave) * K_T0) / D;
+        pX[t] = alt * (th - (la.x * mu) * t1) / D;
+        pY[t] = alt * (la.x * mu);
+        if (top) P_lid = 2.f * la.z * c2a * alt * v1;
+        s.t_2[o] = th;
+        if (keep_aux) s.t_2save[o] = v1;
+        A[m * C + col] = c2a * alt * v1;
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const int m = kl + t * KL, k = m + 1;
+      if (m < nz) {
+        const bool top = m == nz - 1;
+        const Off o = ob + k * ni, ow = o + ni, op = top ? ow : ow + ni;
+        const L4 la = LA[m], lap = LA[top ? m : m + 1], lbp = LB[top ? m : m + 1];
+        const float c1f = top ? c1f_top : lbp.x, c2f = top ? c2f_top : lbp.y;
+        const float ph1m = s.ph_save[o], ph1 = s.ph_save[ow], ph1p = s.ph_save[op];
+        const float pbm = s.phb[o], pb0 = s.phb[ow], pbp = s.phb[op];
+        // omega at w levels k, k + 1, k + 2
+        const float ww_hi = W[m * C + col], ww_hh = W[(top ? m : m + 1) * C + col];
+        const float ww_lo = m == 0 ? ww_bot : W[(m - 1) * C + col];
+        const float dph_hi = ph1p - ph1 + pbp - pb0;
+        const float dph_lo = ph1 - ph1m + pb0 - pbm;
+        const float wd_hi = z2 ? lap.z * dph_hi : .5f * (ww_hh + ww_hi) * lap.z * dph_hi;
+        const float wd_lo = z2 ? la.z * dph_lo : .5f * (ww_hi + ww_lo) * la.z * dph_lo;
+        float r = dts * (s.ph_tend[ow] + .5f * K_G * (1.f - epssm) * s.w_2[ow]);
+        if (!top) {
+          if (z2) r = r - dts * ww_hi * (lbp.z * wd_hi + lbp.w * wd_lo);
+          else r = r - dts * (lbp.z * wd_hi + lbp.w * wd_lo);
+        }
+        r = s.ph_2[ow] + msfty * r / (c1f * mut + c2f);
+        if (c.top_lid && top) r = 0.f;
+        R[m * C + col] = r;
+      }
+    }
+  }
+  float q_rw[TASKS], q_cqw[TASKS], q_w[TASKS];
+  if (act) {
+    WRFMI_PHASE;
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const Off o = ob + imin(kl + t * KL + 2, nz + 1) * ni;
+      q_rw[t] = s.rw_tend[o];
+      q_cqw[t] = s.cqw[o];
+      q_w[t] = s.w_2[o];
+    }
+  }
+  __syncthreads();
+
+  // ---- per mass level, the pressure term of the w equation (1402-1431)
+  float e_lid = 0.f;  // the lid equation takes the term itself
+  if (act) {
+    WRFMI_PHASE;
+    const float epssm = a.c.epssm;
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const int m = kl + t * KL;
+      if (m < nz) {
+        const L4 la = LA[m];
+        const float rhs_m = m == 0 ? 0.f : R[(m - 1) * C + col];  // rhs(1) = 0
+        const float e = (1.f + epssm) * (R[m * C + col] - rhs_m) +
+                        (1.f - epssm) * (s.ph_2[ob + (m + 2) * ni] - s.ph_2[ob + (m + 1) * ni]);
+        if (m == nz - 1) e_lid = e;
+        B[m * C + col] = q_c2a[t] * la.z / (la.x * mut + la.y) * e;
+      }
+    }
+  }
+  __syncthreads();
+  // ---- the explicit w
+  float wv[TASKS];
+  if (act) {
+    WRFMI_PHASE;
+    const float dts = a.dts, c1f_top = s.c1f[X1(d, nz + 1)], msft_inv = 1.f / msfty;
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const int m = kl + t * KL, k = m + 2;  // w level
+      if (m < nz - 1) {
+        const float rdn = s.rdn[X1(d, k)];
+        wv[t] = q_w[t] + dts * q_rw[t] +
+                msft_inv * q_cqw[t] * (+.5f * dts * K_G * rdn * (B[(m + 1) * C + col] - B[m * C + col])) +
+                dts * K_G * msft_inv * (rdn * (A[(m + 1) * C + col] - A[m * C + col]) - (LB[m + 1].x * muave));
+      } else if (m == nz - 1) {
+        const L4 la = LA[m];
+        wv[t] = q_w[t] + dts * q_rw[t] +
+                msft_inv * (-.5f * dts * K_G / (la.x * mut + la.y) * (la.z * la.z) * 2.f * q_c2a[t] * e_lid -
+                            dts * K_G * (P_lid + (c1f_top * muave)));
+        if (a.c.top_lid) wv[t] = 0.f;
+      }
+    }
+  }
+  __syncthreads();
+  // ---- calc_coef_w's coefficients (570-652)
+  if (act) {
+    WRFMI_PHASE;
+    const CT lid = a.c.top_lid ? CT(0) : CT(1), epc = (CT)a.c.epssm, MUT = (CT)mut;
+    CT cof = (CT(.5) * (CT)a.dts * (CT)K_G * (CT(1) + epc));
+    cof = cof * cof;
+    const float c1f_top = s.c1f[X1(d, nz + 1)], c2f_top = s.c2f[X1(d, nz + 1)];
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const int m = kl + t * KL, k = m + 2;  // w level
+      if (m < nz) {
+        const bool top = m == nz - 1;
+        const L4 la = LA[m], lb = LB[m], lap = LA[top ? m : m + 1], lbp = LB[top ? m : m + 1];
+        const L4 lbq = LB[imin(m + 2, nz - 1)];
+        const float c1f = top ? c1f_top : lbp.x, c2f = top ? c2f_top : lbp.y;
+        const CT cHm = (CT)la.x * MUT + (CT)la.y, cFm = (CT)lb.x * MUT + (CT)lb.y, cF = (CT)c1f * MUT + (CT)c2f;
+        const CT C2Al = (CT)q_c2a[t];
+        CT wa, wb, wc;
+        if (!top) {
+          const float c1f_n = m + 2 < nz ? lbq.x : c1f_top, c2f_n = m + 2 < nz ? lbq.y : c2f_top;
+          const CT rdn = (CT)s.rdn[X1(d, k)], CQW = (CT)q_cqw[t], C2A = (CT)s.c2a[ob + k * ni];
+          const CT cH = (CT)lap.x * MUT + (CT)lap.y, cFp = (CT)c1f_n * MUT + (CT)c2f_n;
+          wa = k >= 3 ? -CQW * cof * rdn * (CT)la.z * C2Al / (cHm * cFm) : CT(0);
+          wb = CT(1) + CQW * cof * rdn * ((CT)lap.z * C2A / (cH * cF) + (CT)la.z * C2Al / (cHm * cF));
+          wc = -CQW * cof * rdn * (CT)lap.z * C2A / (cH * cFp);
+        } else {
+          wa = -CT(2) * cof * ((CT)la.z * (CT)la.z) * C2Al * lid / (cHm * cFm);
+          wb = CT(1) + CT(2) * cof * ((CT)la.z * (CT)la.z) * C2Al / (cHm * cF);
+          wc = CT(0);
+        }
+        Q[m * C + col] = Row<CT>{wa, wb, wc, (CT)wv[t]};
+      }
+    }
+  }
+  float q_pm1[TASKS];
+  if (act) {
+    WRFMI_PHASE;
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) q_pm1[t] = s.pm1[ob + imin(kl + t * KL + 1, nz) * ni];
+  }
+  __syncthreads();
+
+  // ---- the tridiagonal sweeps (1433-1443)
+  if (serial) {
+    CT gam = CT(0), wfe = (CT)wsfc;
+    sweep_up<CT, C>(Q + col, nz, gam, wfe);
+    CT wup = wfe;
+    serial_up<2, CT>(
+        nz - 1, [&](int f, int m) { return f == 0 ? Q[(nz - 2 - m) * C + col].c : Q[(nz - 2 - m) * C + col].w; },
+        [&](int m, const CT *y) {
+          wup = y[1] - y[0] * wup;
+          Q[(nz - 2 - m) * C + col].w = wup;
+        });
+  }
+  __syncthreads();
+
+  // ---- the w damping layer (1445-1458), ph and calc_p_rho
+  if (act) {
+    WRFMI_PHASE;
+    const wrfmi_config &c = a.c;
+    const bool damp3 = c.damp_opt == 3, keep_aux = a.keep & kKeepAux;
+    const float dts = a.dts, epssm = c.epssm, dampmag = dts * c.dampcoef, hdepth = c.zdamp;
+    const float c1f_top = s.c1f[X1(d, nz + 1)], c2f_top = s.c2f[X1(d, nz + 1)];
+    const float htop = damp3 ? (s.ph_save[ob + (nz + 1) * ni] + s.phb[ob + (nz + 1) * ni]) / K_G : 0.f;
+    FPtr<CT> GA((CT *)s.gamma);
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const int m = kl + t * KL, k = m + 2;
+      if (m < nz) {
+        const Off o = ob + k * ni;
+        const L4 lbp = LB[imin(m + 1, nz - 1)];
+        const float c1f = m < nz - 1 ? lbp.x : c1f_top, c2f = m < nz - 1 ? lbp.y : c2f_top;
+        float wk = (float)Q[m * C + col].w;
+        if (keep_aux && k <= nz) GA[o] = Q[m * C + col].c;
+        if (damp3) {
+          const float hk = (s.ph_save[o] + s.phb[o]) / K_G;
+          const float hbot = htop - hdepth;
+          float dampwt = 0.f;
+          if (hk >= hbot) {
+            const float sn = (float)sin((double)(.5f * (4.f * 0.785398185f) * (hk - hbot) / hdepth));
+            dampwt = dampmag * sn * sn;
+          }
+          wk = (wk - dampwt * (c1f * mut + c2f) * s.w_save[o]) / (1.f + dampwt);
+        }
+        const float phk = R[m * C + col] + msfty * .5f * dts * K_G * (1.f + epssm) * wk / (c1f * muts + c2f);
+        s.w_2[o] = wk;
+        s.ph_2[o] = phk;
+        R[m * C + col] = phk;
+      }
+    }
+  }
+  __syncthreads();
+  if (act) {
+    WRFMI_PHASE;
+    const float smdiv = a.c.smdiv;
+#pragma unroll
+    for (int t = 0; t < TASKS; t++) {
+      const int m = kl + t * KL;
+      if (m < nz) {
+        const Off o = ob + (m + 1) * ni;
+        const L4 la = LA[m];
+        const float ph_lo = m == 0 ? s.ph_2[ob + ni] : R[(m - 1) * C + col];
+        const float al = -1.f / (la.x * muts + la.y) * (pY[t] + la.z * (R[m * C + col] - ph_lo));
+        s.al[o] = al;
+        float pp = q_c2a[t] * (pX[t] - al);
+        const float ptmp = pp;
+        pp = pp + smdiv * (pp - q_pm1[t]);
+        s.p[o] = pp;
+        s.pm1[o] = ptmp;
+      }
+    }
+  }
+}
+
+#define WRFMI_INST_COL(C, TASKS) \
+  template __global__ void k_ac_column<KArgs, float, false, C, TASKS>(KArgs); \
+  template __global__ void k_ac_column<BatchArgs, float, false, C, TASKS>(BatchArgs); \
+  template __global__ void k_ac_column<KArgs, double, true, C, TASKS>(KArgs); \
+  template __global__ void k_ac_column<BatchArgs, double, true, C, TASKS>(BatchArgs);
+WRFMI_COL_SHAPES(WRFMI_INST_COL)
+
+}  // namespace wrfmi

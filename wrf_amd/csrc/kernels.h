@@ -20,6 +20,33 @@ constexpr int kPdVK = 4;       // levels per thread in k_pd_scale_x4 and k_pd_te
 // taller tile re-reads fewer of the j+-3 halo rows its stencils share with the tiles above
 // and below.  (At 1024 threads the compiler would cap them at 128 VGPRs and spill.)
 constexpr int kTallBlk = 512;
+// k_ac_column: kColThreads threads take a tile of C columns of one row, C lanes along i by
+// kColThreads / C level lanes, each lane up to `tasks` levels.  The compiled shapes, and the
+// levels each holds (fewer threads than 512, or a count that is no multiple of four waves,
+// measured slower for the same levels: a barrier then waits for the SIMD with the extra wave):
+//   C   tasks  levels
+#define WRFMI_COL_SHAPES(X) \
+  X(32, 3) /* 48 */ \
+  X(32, 4) /* 64 */ \
+  X(32, 5) /* 80 */ \
+  X(16, 2) /* 64 */ \
+  X(16, 3) /* 96 */ \
+  X(16, 5) /* 160 */ \
+  X(8, 3)  /* 192 */ \
+  X(8, 5)  /* 320 */
+constexpr int kColThreads = 512;
+struct ColShape {
+  int c, tasks;  // c == 0: no shape holds the columns
+};
+// LDS of a tile: per level and column four values of the coefficient type and a float, per
+// level eight coefficients
+HDI size_t col_lds(int c, int nz, bool p64) { return (size_t)nz * (c * (4 * (p64 ? 8 : 4) + 4) + 32); }
+// First i of k_ac_column's tiles: ids rounded down to C points of the row (whole cache lines
+// for C = 32), unless that takes one more tile to cover the mass columns.
+HDI int col_tile_ia(const Dm &d, int C) {
+  const int ia = d.ims + ((d.ids - d.ims) & ~(C - 1));
+  return (d.ide - ia + C - 1) / C == (d.ide - d.ids + C - 1) / C ? ia : d.ids;
+}
 // The reference routine a launch computes on its own, for the per-routine entry points
 // with the reference's argument lists (KArgs::routine); R_FUSED is the whole step's form,
 // with each kernel's fused parts.
@@ -59,6 +86,7 @@ template <typename A> __global__ void k_small_prep_x4(A);
 template <typename A> __global__ void k_p_rho0_x4(A);
 template <typename A> __global__ void k_ac_theta_x4(A);
 template <typename A, typename CT, bool PRHO = true, int PF = 4> __global__ void k_ac_wsolve(A);
+template <typename A, typename CT, bool COMP, int C, int TASKS> __global__ void k_ac_column(A);
 template <typename A> __global__ void k_calc_p_rho(A);
 template <typename A> __global__ void k_small_finish(A);
 template <typename A> __global__ void k_small_finish_x4(A);

@@ -358,13 +358,13 @@ enum KernelId {
   KID_STEP_PREP, KID_TEND_U, KID_TEND_V, KID_TEND_W, KID_TEND_T, KID_SMALL_PREP, KID_ADVANCE_UV,
   KID_AC_DIV, KID_SMALL_FINISH, KID_ADV_SCALAR, KID_UPDATE_SCALAR, KID_P_RHO_PHI, KID_HALO, KID_P_RHO0,
   KID_COEF_W, KID_WW_SCAN, KID_AC_MU_WW, KID_AC_THETA, KID_AC_WSOLVE, KID_W_SURFACE, KID_PD_SCALE, KID_PD_TEND,
-  KID_UPDATE_SCALAR_PD, KID_DIFF6, KID_RAYLEIGH, KID_DIFF2, KID_LBC, KID_COUNT
+  KID_UPDATE_SCALAR_PD, KID_DIFF6, KID_RAYLEIGH, KID_DIFF2, KID_LBC, KID_AC_COLUMN, KID_COUNT
 };
 static const char *kKernelNames[KID_COUNT] = {
   "k_step_prep", "k_tend_u", "k_tend_v", "k_tend_w", "k_tend_t", "k_small_prep", "k_advance_uv",
   "k_ac_div", "k_small_finish", "k_adv_scalar", "k_update_scalar", "k_p_rho_phi", "k_halo", "k_p_rho0",
   "k_coef_w", "k_ww_scan", "k_ac_mu_ww", "k_ac_theta", "k_ac_wsolve", "k_set_w_surface", "k_pd_scale", "k_pd_tend",
-  "k_update_scalar_pd", "k_diff6", "k_rayleigh", "k_diff2", "k_lbc"};
+  "k_update_scalar_pd", "k_diff6", "k_rayleigh", "k_diff2", "k_lbc", "k_ac_column"};
 struct EvPair { int id; hipEvent_t a, b; };
 static unsigned g_timing = 0;  // bit n set: time launches of kernel n
 static std::vector<EvPair> g_ev_pending;
@@ -392,6 +392,7 @@ struct KRef {
 #define KRP(K, P) KRef{K<KArgs, P>, K<BatchArgs, P>}
 #define KRZ(K) KRef{K<KArgs, false, true>, K<BatchArgs, false, true>}
 #define KRC(K, P, Q) KRef{K<KArgs, P, Q>, K<BatchArgs, P, Q>}
+#define KRCOL(CT, COMP, C, T) KRef{k_ac_column<KArgs, CT, COMP, C, T>, k_ac_column<BatchArgs, CT, COMP, C, T>}
 #define KRWS(CT, PF) KRef{k_ac_wsolve<KArgs, CT, true, PF>, k_ac_wsolve<BatchArgs, CT, true, PF>}
 
 // One launch of an ensemble member, as recorded for a batched launch (wrfmi_ensemble_*).
@@ -402,6 +403,7 @@ struct RecOp {
   dim3 blk;
   unsigned wgs;    // workgroups of this member
   size_t arg;      // index into RecMember::k or ::h
+  size_t lds;      // dynamic LDS of a workgroup
 };
 struct RecMember {
   std::vector<RecOp> ops;
@@ -429,36 +431,41 @@ struct Launcher {
   bool vec = false;          // the layout allows the four-points-per-lane kernels
   bool scal_all = false;     // species advected and updated by the all-species kernels
   bool zone_ok = false;      // each open direction is wide enough for a boundary zone on each side
+  ColShape col{0, 0};        // tiles of k_ac_column; c == 0: its four routine kernels instead
   bool whole_step = false;   // enqueued by the whole-step driver (work arrays stay internal)
   bool lbc_on = false;       // specified boundaries: lbc holds the boundary arrays' device addresses
   wrfmi_lbc lbc;
   // launch with an optional event pair around it (kernel timing mode)
   template <typename K, typename... A>
   void launch(int id, K kern, dim3 g, dim3 b, A... args) {
+    launch_lds(id, kern, g, b, 0, args...);
+  }
+  template <typename K, typename... A>
+  void launch_lds(int id, K kern, dim3 g, dim3 b, size_t lds, A... args) {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (g_timing & (1u << id)) {
       e0 = ev_get();
       e1 = ev_get();
       if (e0 && e1) (void)hipEventRecord(e0, st);
     }
-    hipLaunchKernelGGL(kern, g, b, 0, st, args...);
+    hipLaunchKernelGGL(kern, g, b, (unsigned)lds, st, args...);
     if (e0 && e1) {
       (void)hipEventRecord(e1, st);
       g_ev_pending.push_back(EvPair{id, e0, e1});
     }
   }
   // a state kernel on a tnx x tny x tnz tile grid, launched 1-D for the XCD-aware order
-  void launchK(int id, KRef kern, dim3 g, dim3 b, KArgs args) {
+  void launchK(int id, KRef kern, dim3 g, dim3 b, KArgs args, size_t lds = 0) {
     args.tnx = (int)g.x;
     args.tny = (int)g.y;
     args.tnz = (int)g.z;
     const unsigned n = g.x * g.y * g.z;
     if (rec) {
-      rec->ops.push_back(RecOp{id, false, (void *)kern.batch, b, n, rec->k.size()});
+      rec->ops.push_back(RecOp{id, false, (void *)kern.batch, b, n, rec->k.size(), lds});
       rec->k.push_back(args);
       return;
     }
-    launch(id, kern.one, dim3(n, 1, 1), b, args);
+    launch_lds(id, kern.one, dim3(n, 1, 1), b, lds, args);
   }
   void halo_begin() { h.n = 0; }
   void halo_add(float *p, char kind, int is3d) {
@@ -474,7 +481,7 @@ struct Launcher {
     const long nthreads = ring * ((d.kde + kHaloK - 1) / kHaloK) * h.n;
     const unsigned wgs = (unsigned)((nthreads + 255) / 256);
     if (rec) {
-      rec->ops.push_back(RecOp{KID_HALO, true, (void *)k_halo<BatchHalo>, dim3(256, 1, 1), wgs, rec->h.size()});
+      rec->ops.push_back(RecOp{KID_HALO, true, (void *)k_halo<BatchHalo>, dim3(256, 1, 1), wgs, rec->h.size(), 0});
       rec->h.push_back(h);
     } else {
       launch(KID_HALO, k_halo<HaloArgs>, dim3(wgs, 1, 1), dim3(256, 1, 1), h);
@@ -500,7 +507,7 @@ static Shape default_shape(int kid) {
 // which of a kernel's shape parameters are tunable, and the values each may take
 static bool tunable_rows(int kid) {
   return kid != KID_HALO && kid != KID_W_SURFACE && kid != KID_PD_SCALE && kid != KID_PD_TEND && kid != KID_UPDATE_SCALAR_PD &&
-         kid != KID_DIFF6 && kid != KID_RAYLEIGH && kid != KID_DIFF2 && kid != KID_LBC;
+         kid != KID_DIFF6 && kid != KID_RAYLEIGH && kid != KID_DIFF2 && kid != KID_LBC && kid != KID_AC_COLUMN;
 }
 static bool tunable_levels(int kid) { return kid == KID_ADVANCE_UV || kid == KID_AC_DIV; }
 // the four-point stencil kernels built for workgroups of up to kTallBlk threads
@@ -568,6 +575,32 @@ static int tune_load(const char *path) {
   fclose(f);
   if (rc) g_tune = saved;
   return rc;
+}
+
+// The tiles of k_ac_column for a launch over ncol mass columns of nz levels.  The widest tile
+// that three workgroups' LDS allows on a CU (else two, else one): 32 columns make a whole
+// cache line of every level's row (80 levels, 400x400 columns: 480 us with 32 columns, 603
+// with 16).  16 columns of two levels a lane where they take less time in all: a CU holds
+// three workgroups of the wide tiles and four of these, whose rounds take about 0.8 of the
+// time (64 levels at most).  Small domains of one round gain (41x41x40: 20.3 against 22.9 us)
+// and those that just begin a second one (200x150x50: 63 against 72), ordinary ones lose
+// (256x256x60: 201 against 167).
+static ColShape col_shape(long ncol, int nz, bool p64) {
+  constexpr long kCUs = 256;
+  ColShape best{0, 0};
+  for (size_t share = 3; share >= 1 && !best.c; share--) {
+#define COL_FITS(C, T) \
+  if (!best.c && T * (kColThreads / C) >= nz && share * col_lds(C, nz, p64) <= 160 * 1024 && \
+      col_lds(C, nz, p64) <= 64 * 1024) \
+    best = ColShape{C, T};
+    WRFMI_COL_SHAPES(COL_FITS)
+#undef COL_FITS
+  }
+  if (best.c == 32 && nz <= 64) {
+    const long wide = (ncol / 32 + 3 * kCUs - 1) / (3 * kCUs), narrow = (ncol / 16 + 4 * kCUs - 1) / (4 * kCUs);
+    if (4 * narrow < 5 * wide) best = ColShape{16, 2};
+  }
+  return best;
 }
 
 // ------------------------------------------------------------------ phases of one RK substep
@@ -821,9 +854,10 @@ static void ph_advance_uv(Launcher &L) {
                {lbc_job('u', s.u_2, nullptr, s.ru_tend), lbc_job('v', s.v_2, nullptr, s.rv_tend)});
   }
 }
-static void ph_advance_mu_t_w(Launcher &L) {
+// advance_mu_t, advance_w, sumflux and calc_p_rho by their routine kernels, for columns too
+// tall for k_ac_column's LDS
+static void ac_routines(Launcher &L) {
   const KArgs &a = L.a;
-  const wrfmi_state &s = a.s;
   const bool p64 = a.c.precision_mode == 1;
   const int nk = a.d.kde - a.d.kds + 1;
   if (L.vec) {
@@ -836,17 +870,39 @@ static void ph_advance_mu_t_w(Launcher &L) {
   else L.launchK(KID_AC_MU_WW, KRP(k_ac_mu_ww, false), gcol(L, KID_AC_MU_WW), cblk(L, KID_AC_MU_WW), a);
   if (L.vec) L.launchK(KID_AC_THETA, KR(k_ac_theta_x4), gvec(L, KID_AC_THETA, nk), vblk(L, KID_AC_THETA), a);
   else L.launchK(KID_AC_THETA, KR(k_ac_theta), g_pt3(a.d, nk), kColBlk, a);
+  const int pf = L.sh[KID_AC_WSOLVE].prefetch;
+  KRef k;
+  if (p64) k = pf == 2 ? KRWS(double, 2) : pf == 8 ? KRWS(double, 8) : KRWS(double, 4);
+  else k = pf == 2 ? KRWS(float, 2) : pf == 8 ? KRWS(float, 8) : KRWS(float, 4);
+  L.launchK(KID_AC_WSOLVE, k, gcol(L, KID_AC_WSOLVE), cblk(L, KID_AC_WSOLVE), a);
+}
+static void ph_advance_mu_t_w(Launcher &L) {
+  KArgs &a = L.a;
+  const wrfmi_state &s = a.s;
+  if (L.col.c) {
+    const bool p64 = a.c.precision_mode == 1;
+    const ColShape &cs = L.col;
+    const int ia = col_tile_ia(a.d, cs.c);
+    // the whole step needs omega after an RK substep's last acoustic step, and leaves t_2save
+    // and gamma as the step's last acoustic step does; a per-routine call leaves them all
+    const bool end = a.iteration == a.nsmall;
+    a.keep = !L.whole_step ? kKeepWW | kKeepAux : end ? kKeepWW | (a.rk_step == 3 ? kKeepAux : 0) : 0;
+    KRef k{nullptr, nullptr};
+#define COL_IS(C, T) \
+  if (cs.c == C && cs.tasks == T) k = p64 ? KRCOL(double, true, C, T) : KRCOL(float, false, C, T);
+    WRFMI_COL_SHAPES(COL_IS)
+#undef COL_IS
+    L.launchK(KID_AC_COLUMN, k, dim3((a.d.ide - ia + cs.c - 1) / cs.c, a.d.jde - a.d.jds + 1, 1),
+              dim3(cs.c, kColThreads / cs.c, 1), a, col_lds(cs.c, a.d.kde - a.d.kds, p64));
+  } else {
+    ac_routines(L);
+  }
+  // the specified boundaries' updates touch their frame of columns only, which the kernels
+  // above leave out
   if (L.lbc_on) {  // spec_bdyupdate of theta, mu and muts (solve_em.F:1459-1490)
     lbc_launch(L, LBC_UPDATE, a.dts, 0, a.c.spec_zone,
                {lbc_job('t', s.t_2, nullptr, s.t_tend), lbc_job('m', s.mu_2, nullptr, s.mu_tend),
                 lbc_job('m', s.muts, nullptr, s.mu_tend)});
-  }
-  {
-    const int pf = L.sh[KID_AC_WSOLVE].prefetch;
-    KRef k;
-    if (p64) k = pf == 2 ? KRWS(double, 2) : pf == 8 ? KRWS(double, 8) : KRWS(double, 4);
-    else k = pf == 2 ? KRWS(float, 2) : pf == 8 ? KRWS(float, 8) : KRWS(float, 4);
-    L.launchK(KID_AC_WSOLVE, k, gcol(L, KID_AC_WSOLVE), cblk(L, KID_AC_WSOLVE), a);
   }
   if (L.lbc_on && a.c.non_hydrostatic) {
     // spec_bdyupdate_ph, zero_grad_bdy of w (solve_em.F:1583-1620), and calc_p_rho on the
@@ -1145,6 +1201,7 @@ static int prepare(const wrfmi_state *st_in, const wrfmi_config *cfg, const wrfm
   // ensemble members are recorded with the default shapes (one launch sequence for all)
   for (int k = 0; k < KID_COUNT; k++) L.sh[k] = default_shapes ? default_shape(k) : shape_for(k, d);
   L.vec = vec_layout(s, d, L.a);
+  L.col = col_shape((long)(d.ide - d.ids) * (d.jde - d.jds), d.kde - d.kds, cfg->precision_mode == 1);
   // the all-species scalar kernels (doubly periodic, aligned layout, more than one species)
   L.scal_all = L.vec && cfg->periodic_x && cfg->periodic_y && s.n_species > 1 && (own_qt || !own_scratch);
   L.zone_ok = (cfg->periodic_x || d.ide - d.ids + 1 >= 2 * kZone + 2) && (cfg->periodic_y || d.jde - d.jds + 1 >= 2 * kZone + 2);
@@ -1321,6 +1378,7 @@ struct EnsOp {
   void *kern;
   dim3 blk;
   unsigned total;
+  size_t lds;
   BatchArgs ka;
   BatchHalo ha;
 };
@@ -1397,12 +1455,22 @@ extern "C" int wrfmi_ensemble_create(int n_members, const wrfmi_state *states, c
   // member's layout allows them
   bool all_vec = true;
   for (int m = 0; m < n_members && !rc; m++) all_vec = all_vec && Ls[m].vec;
+  // ... and k_ac_column's tiles: one shape, which the tallest member's columns fit
+  int nz_max = 0;
+  long ncol = 0;
+  for (int m = 0; m < n_members && !rc; m++) {
+    const Dm &d = Ls[m].a.d;
+    nz_max = d.kde - d.kds > nz_max ? d.kde - d.kds : nz_max;
+    ncol += (long)(d.ide - d.ids) * (d.jde - d.jds);
+  }
+  const ColShape col = col_shape(ncol, nz_max, cfgs[0].precision_mode == 1);
   bool all_zone = true;
   for (int m = 0; m < n_members && !rc; m++) all_zone = all_zone && Ls[m].zone_ok;
   for (int m = 0; m < n_members && !rc; m++) {
     Ls[m].vec = all_vec;
     Ls[m].scal_all = Ls[m].scal_all && all_vec;
     Ls[m].zone_ok = all_zone;
+    Ls[m].col = col;
     Ls[m].rec = &rec[m];
     enqueue_step(Ls[m]);
   }
@@ -1462,7 +1530,9 @@ extern "C" int wrfmi_ensemble_create(int n_members, const wrfmi_state *states, c
     }
     unsigned total = 0;
     for (unsigned v : w) total += v;
-    EnsOp eo{op0.id, op0.halo, op0.kern, op0.blk, total, {}, {}};
+    size_t lds = 0;
+    for (int m = 0; m < n_members; m++) lds = rec[m].ops[o].lds > lds ? rec[m].ops[o].lds : lds;
+    EnsOp eo{op0.id, op0.halo, op0.kern, op0.blk, total, lds, {}, {}};
     e->ops.push_back(eo);
     pend.push_back(Pending{ao, it->second.first, it->second.second});
   }
@@ -1489,7 +1559,7 @@ static void ens_enqueue(wrfmi_ensemble *e, hipStream_t st) {
   L.st = st;
   for (const EnsOp &o : e->ops) {
     if (o.halo) L.launch(o.id, (void (*)(BatchHalo))o.kern, dim3(o.total, 1, 1), o.blk, o.ha);
-    else L.launch(o.id, (void (*)(BatchArgs))o.kern, dim3(o.total, 1, 1), o.blk, o.ka);
+    else L.launch_lds(o.id, (void (*)(BatchArgs))o.kern, dim3(o.total, 1, 1), o.blk, o.lds, o.ka);
   }
 }
 static bool ens_known(wrfmi_ensemble *e) {
