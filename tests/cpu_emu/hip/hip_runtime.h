@@ -83,6 +83,7 @@ inline unsigned __float_as_uint(float x) {
   std::memcpy(&u, &x, 4);
   return u;
 }
+inline unsigned __umulhi(unsigned a, unsigned b) { return (unsigned)(((unsigned long long)a * b) >> 32); }
 typedef void *hipDeviceptr_t;
 hipError_t hipMemGetAddressRange(hipDeviceptr_t *base, size_t *size, hipDeviceptr_t p);
 inline hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }

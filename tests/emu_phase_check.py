@@ -84,6 +84,12 @@ CASES = {
     "col_16": dict(nx=17, ny=7, nz=97, bc="periodic", n_bubbles=1, seed=65),
     "col_8": dict(nx=9, ny=7, nz=193, bc="periodic", n_bubbles=1, seed=66),
     "col_tall": dict(nx=9, ny=7, nz=321, bc="open", n_bubbles=1, seed=67),
+    # rows of 2, 3, 10, 16 and 17 four-point groups, which the four-point kernels' waves run across
+    "vec_7": dict(nx=7, ny=33, nz=5, bc="periodic", n_bubbles=1, seed=71, pd=(1, 1)),
+    "vec_8": dict(nx=8, ny=44, nz=5, bc="periodic", n_passive=1, n_bubbles=1, seed=72),
+    "vec_36": dict(nx=36, ny=13, nz=5, bc="open", n_bubbles=1, seed=73),
+    "vec_63": dict(nx=63, ny=9, nz=5, bc="periodic", n_passive=1, n_bubbles=1, seed=74),
+    "vec_64": dict(nx=64, ny=9, nz=5, bc="specified", n_passive=1, n_bubbles=1, seed=75, lbc=55, pd=(1, 1)),
     "pd_mixed_unaligned": dict(nx=14, ny=11, nz=8, bc_x="open", bc_y="periodic", n_passive=1, n_bubbles=1, seed=28,
                                pad_i=1, pd=(0, 1)),
 }

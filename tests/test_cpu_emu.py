@@ -53,6 +53,16 @@ def test_emulated_column_tiles_match_oracle(emu_env, case, order):
     assert "OK" in r.stdout
 
 
+@pytest.mark.parametrize("case,order", [("vec_7", 1), ("vec_8", 0), ("vec_36", 1), ("vec_63", 0), ("vec_64", 1)])
+def test_emulated_four_point_rows_match_oracle(emu_env, case, order):
+    """The four-point kernels' waves across the ends of rows of few groups, bit for bit with
+    the oracle."""
+    r = subprocess.run([sys.executable, os.path.join(HERE, "emu_phase_check.py"), case, str(order), "1"],
+                       env=emu_env, capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-4000:]
+    assert "OK" in r.stdout
+
+
 def test_emulated_host_array_registry(emu_env):
     r = subprocess.run([sys.executable, os.path.join(HERE, "emu_phase_check.py"), "registry"],
                        env=emu_env, capture_output=True, text=True, timeout=300)

@@ -122,6 +122,11 @@ struct KArgs {
   float *scr_qt;        // advect_tend of species 0 .. n_species-2 (all-species scalar kernels),
   unsigned long long qt_stride;  // one grid field (elements) apart
   int tnx, tny, tnz;  // tiles of the current launch in i, j and k (see tile3)
+  // four-point launches (see vec_ij): groups of four points per row, 2^32 / vg, and the first
+  // group's i and j
+  int vg;
+  unsigned vmagic;
+  int vi0, vj0;
   int routine;        // Routine: R_FUSED in the whole step and the grouped entry points
   int keep;           // k_ac_column: the column work it stores for its callers (kKeep*)
 };
@@ -260,6 +265,25 @@ template <typename T> DEVI T imax(T a, T b) { return a > b ? a : b; }
 // Vector kernels: a lane holds the four points i0..i0+3, where i0 - ims is a multiple of four
 // (so that the lane's memory is a 16-byte group); vec_ia0 is the first such i at or below ids.
 HDI int vec_ia0(const Dm &d) { return d.ims + 4 * ((d.ids - d.ims) >> 2); }
+// The lane's group of four points.  Wave y of a workgroup takes row y of a band of blockDim.y
+// rows, and the groups of all bands form one sequence, 64 after 64, so that a wave goes on with
+// the next band where a row ends.  With a wave per 256 points of one row, the staggered point
+// ide alone began a second wave on rows of 256 points, and rows of 41 left 83 % of the lanes
+// idle.  Per launch, a wave per row against this: k_tend_v_x4 117 and 93 us at 256x256x60,
+// 44 and 38 at 160x128x80, k_p_rho_phi_x4 157 and 130 at 400x400x80; the 64-member ensemble's
+// step 105.2 and 98.6 ms.  (A sequence of all rows without bands loses the rows that the stencils
+// in j share within a workgroup.)
+// The quotient by the reciprocal vmagic is one too small at most.
+DEVI void vec_ij(const KArgs &a, const Tile3 &T, int &i0, int &j) {
+  const unsigned n = (unsigned)T.bx * 64u + threadIdx.x;
+  unsigned q = __umulhi(n, a.vmagic), r = n - q * (unsigned)a.vg;
+  if (r >= (unsigned)a.vg) {
+    q++;
+    r -= (unsigned)a.vg;
+  }
+  i0 = a.vi0 + 4 * (int)r;
+  j = a.vj0 + (int)(q * blockDim.y + threadIdx.y);
+}
 // store of the lane's points that lie in [lo, hi]
 DEVI void st4m(const FPtr<float> &p, Off o, const F4 &v, int i0, int lo, int hi) {
   if (i0 >= lo && i0 + 3 <= hi) {

@@ -430,8 +430,8 @@ __global__ void __launch_bounds__(256) k_pd_scale_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int kts = d.kds, ktf = d.kde - 1;
   const int k0 = kts + T.bz * kPdVK, k1 = imin(k0 + kPdVK - 1, ktf);
   if (i0 > d.ide - 1 || j > d.jde - 1 || k0 > ktf) return;
@@ -489,8 +489,8 @@ __global__ void __launch_bounds__(256) k_pd_tend_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int kts = d.kds, kte = d.kde, ktf = kte - 1;
   const int k0 = kts + T.bz * kPdVK, k1 = imin(k0 + kPdVK - 1, kte);
   if (i0 > d.ide || j > d.jde || k0 > kte) return;

@@ -121,8 +121,8 @@ __global__ void __launch_bounds__(256) k_step_prep_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) - 4 + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds - 1 + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int k = d.kds + (int)T.bz;
   const int ids = d.ids, ide = d.ide, jds = d.jds, jde = d.jde, kde = d.kde;
   if (i0 > ide || j > jde || k > kde) return;

@@ -157,9 +157,8 @@ __global__ void __launch_bounds__(kTallBlk) k_adv_scalar_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int ia0 = d.ims + 4 * ((d.ids - d.ims) >> 2);
-  const int i0 = ia0 + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int k0 = d.kds + T.bz * kAdvVK;
   const int ids = d.ids, ide = d.ide, jde = d.jde, kts = d.kds, kte = d.kde, ktf = kte - 1;
   if (i0 > ide || j > jde || !zrow(a, j)) return;  // rows of an open y edge: the zone form
@@ -173,7 +172,7 @@ __global__ void __launch_bounds__(kTallBlk) k_adv_scalar_x4(ARGS args) {
   const Off ob = X3(d, i0, 0, j);  // level k at ob + k*ni
   auto at = [&](int k) { return ob + k * ni; };
   const F4 msftx = s.msftx.ld<F4>(X2(d, i0, j));
-  const bool jmass = j <= jde - 1;
+  const int imass = j <= jde - 1 ? ide - 1 : i0 - 1;  // the row's last mass point, from the lane's first
   // vertical flux at w level kp from q at kp-2..kp+1 (vflux of k_adv_scalar)
   auto vflux = [&](int kp, const F4 &qm2, const F4 &qm1, const F4 &q0, const F4 &qp1, const F4 &w) {
     const float fm = s.fnm[X1(d, imin(kp, kte))], fp = s.fnp[X1(d, imin(kp, kte))];
@@ -218,6 +217,7 @@ __global__ void __launch_bounds__(kTallBlk) k_adv_scalar_x4(ARGS args) {
     }
     const F4 vf_hi = vflux(k + 1, qm1, q0, qp1, qp2, wp);
     const float rdnw = s.rdnw[X1(d, imin(k, ktf))];
+    const int ilast = k <= ktf ? imass : i0 - 1;
     F4 t;
 #pragma unroll
     for (int n = 0; n < 4; n++) {
@@ -227,8 +227,7 @@ __global__ void __launch_bounds__(kTallBlk) k_adv_scalar_x4(ARGS args) {
       tt = tt - msftx.v[n] * rdy * (fy1 - fy0);
       tt = tt - msftx.v[n] * rdx * (fx[n + 1] - fx[n]);
       tt = tt - rdnw * (vf_hi.v[n] - vf_lo.v[n]);
-      const bool mass = jmass && i0 + n <= ide - 1 && k <= ktf;
-      t.v[n] = mass ? tt : 0.f;
+      t.v[n] = i0 + n <= ilast ? tt : 0.f;
     }
     qm1 = q0;
     q0 = qp1;
@@ -284,8 +283,8 @@ __global__ void __launch_bounds__(kTallBlk) k_adv_scalar_all_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int k = d.kds + (int)T.bz;
   const int ids = d.ids, ide = d.ide, jde = d.jde, kts = d.kds, kte = d.kde, ktf = kte - 1;
   if (i0 > ide || j > jde || k > kte) return;
@@ -307,7 +306,7 @@ __global__ void __launch_bounds__(kTallBlk) k_adv_scalar_all_x4(ARGS args) {
     const float hi = w * flux3(qm2, qm1, q0, qp1, -w, ts);
     return zero ? 0.f : (low ? lo : hi);
   };
-  const bool jmass = j <= jde - 1;
+  const int ilast = j <= jde - 1 && k <= ktf ? ide - 1 : i0 - 1;  // the lane's last mass point
   const int ns = s.n_species;
   for (int m = 0; m < ns; m++) {
     const FPtr<float> f = s.q[m];
@@ -339,8 +338,7 @@ __global__ void __launch_bounds__(kTallBlk) k_adv_scalar_all_x4(ARGS args) {
       tt = tt - msftx.v[n] * rdy * (fy1 - fy0);
       tt = tt - msftx.v[n] * rdx * (fx[n + 1] - fx[n]);
       tt = tt - rdnw * (vf_hi - vf_lo);
-      const bool mass = jmass && i0 + n <= ide - 1 && k <= ktf;
-      t.v[n] = mass ? tt : 0.f;
+      t.v[n] = i0 + n <= ilast ? tt : 0.f;
     }
     const FPtr<float> dst = m == ns - 1 ? s.advect_tend : FPtr<float>(a.scr_qt + (size_t)m * a.qt_stride);
     st4m(dst, os, t, i0, ids, ide);
@@ -355,8 +353,8 @@ __global__ void __launch_bounds__(256) k_update_scalar_all_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int k = d.kds + (int)T.bz;
   if (i0 > d.ide - 1 || j > d.jde - 1 || k > d.kde - 1) return;
   const Off o = X3(d, i0, k, j), o2 = X2(d, i0, j);
@@ -391,8 +389,8 @@ __global__ void __launch_bounds__(256) k_update_scalar_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int k = d.kds + (int)T.bz;
   if (i0 > d.ide - 1 || j > d.jde - 1 || k > d.kde - 1) return;
   const Off o = X3(d, i0, k, j), o2 = X2(d, i0, j);
@@ -423,8 +421,8 @@ __global__ void __launch_bounds__(256) k_p_rho_phi_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int k = d.kds + (int)T.bz;
   if (i0 > d.ide - 1 || j > d.jde - 1 || k > d.kde - 1) return;
   const Off o = X3(d, i0, k, j), o2 = X2(d, i0, j);

@@ -363,8 +363,8 @@ __global__ void __launch_bounds__(256) k_advance_uv_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int k0 = d.kds + (int)T.bz * KS;
   const int ids = d.ids, ide = d.ide, jds = d.jds, jde = d.jde, kde = d.kde;
   const int its = ids, ite = ide, jts = jds, jte = jde;
@@ -699,8 +699,8 @@ __global__ void __launch_bounds__(256) k_small_finish_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int k = d.kds + (int)T.bz;
   const int ids = d.ids, ide = d.ide, jds = d.jds, jde = d.jde, kde = d.kde;
   if (i0 > ide || j > jde || k > kde) return;
@@ -813,8 +813,8 @@ __global__ void __launch_bounds__(256) k_small_prep_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int k = d.kds + (int)T.bz;
   const int ids = d.ids, ide = d.ide, jde = d.jde, kde = d.kde, k_end = kde - 1;
   if (i0 > ide || j > jde || k > kde) return;
@@ -896,8 +896,8 @@ __global__ void __launch_bounds__(256) k_p_rho0_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int k = d.kds + (int)T.bz;
   if (i0 > d.ide - 1 || j > d.jde - 1 || k > d.kde - 1) return;
   if (!a.c.non_hydrostatic) return;
@@ -931,8 +931,8 @@ __global__ void __launch_bounds__(256) k_ac_div_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int k0 = d.kds + (int)T.bz * KS;
   const int ids = d.ids, ide = d.ide, jde = d.jde, kde = d.kde;
   if (i0 > ide || j > jde || k0 > kde) return;
@@ -1001,8 +1001,8 @@ __global__ void __launch_bounds__(256) k_ac_theta_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   const int k = d.kds + (int)T.bz;
   const int ids = d.ids, ide = d.ide, jde = d.jde, kde = d.kde, k_end = kde - 1;
   if (i0 > ide - 1 || j > jde - 1 || k > kde) return;

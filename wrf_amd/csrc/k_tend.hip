@@ -256,8 +256,8 @@ __global__ void __launch_bounds__(kTallBlk) k_tend_u_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   if (!zrow(a, j)) return;  // rows of an open y edge: the zone form
   const int k = d.kds + (int)T.bz;
   const int ids = d.ids, ide = d.ide, jde = d.jde, kde = d.kde, kts = d.kds, kte = kde, ktf = kte - 1;
@@ -650,8 +650,8 @@ __global__ void __launch_bounds__(kTallBlk) k_tend_v_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   if (!zrow(a, j)) return;  // rows of an open y edge: the zone form
   const int k = d.kds + (int)T.bz;
   const int ids = d.ids, ide = d.ide, jde = d.jde, kde = d.kde, kts = d.kds, kte = kde, ktf = kte - 1;
@@ -1038,8 +1038,8 @@ __global__ void __launch_bounds__(kTallBlk) k_tend_w_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   if (!zrow(a, j)) return;  // rows of an open y edge: the zone form
   const int k = d.kds + (int)T.bz;
   const int ids = d.ids, ide = d.ide, jde = d.jde, kde = d.kde, kts = d.kds, kte = kde, ktf = kte - 1;
@@ -1479,8 +1479,8 @@ __global__ void __launch_bounds__(kTallBlk) k_tend_t_x4(ARGS args) {
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i0 = vec_ia0(d) + kVecW * (T.bx * 64 + (int)threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
+  int i0, j;
+  vec_ij(a, T, i0, j);
   if (!zrow(a, j)) return;  // rows of an open y edge: the zone form
   const int k = d.kds + (int)T.bz;
   const int ids = d.ids, ide = d.ide, jde = d.jde, kde = d.kde, kts = d.kds, kte = kde, ktf = kte - 1;

@@ -9,7 +9,6 @@ constexpr int kTendK = 8;    // levels per thread in k_tend_u/v/w/t
 constexpr int kAdvTileI = 63;  // i points per wave in k_adv_scalar (lane 63 supplies a face)
 constexpr int kAdvRows = 4;    // j rows (waves) per block in k_adv_scalar
 constexpr int kVecW = 4;       // i points per lane in the vector kernels (16-byte accesses)
-constexpr int kVecTileI = 64 * kVecW;  // i points per wave in the vector kernels
 constexpr int kAdvVK = 4;      // levels per thread in k_adv_scalar_x4
 constexpr int kHaloK = 8;      // levels per thread in k_halo
 constexpr int kDivK = 4;       // default levels per thread in k_ac_div_x4 (a launch shape)

@@ -330,8 +330,8 @@ static inline dim3 col_grid(const Dm &d, int i0, int j0, dim3 blk) {
   return dim3((ni + blk.x - 1) / blk.x, (nj + blk.y - 1) / blk.y, 1);
 }
 static const dim3 kColBlk(64, 4, 1);
-// workgroup of the four-points-per-lane kernels: one 256-point row per wave, WRFMI_VEC_ROWS
-// rows.  With one row, the tiles of neighbouring rows follow each other more closely in the
+// workgroup of the four-points-per-lane kernels: 64 four-point groups per wave, WRFMI_VEC_ROWS
+// rows (see vec_ij).  With one row, the tiles of neighbouring rows follow each other more closely in the
 // XCD-contiguous tile order, and a launch's waves spread evenly over the CUs: at 400x400x80
 // the step takes 17.45 ms with 1 row, 17.46 with 2 and 17.67 with 4 (8 and 16 were slower
 // still).
@@ -347,7 +347,6 @@ static const dim3 kColBlk(64, 4, 1);
 #ifndef WRFMI_TENDT_ROWS
 #define WRFMI_TENDT_ROWS 4
 #endif
-static const dim3 kVecBlk(64, WRFMI_VEC_ROWS, 1);
 // workgroup of the one-column-per-lane kernels: 64 columns by WRFMI_COL_ROWS rows (see g_col)
 #ifndef WRFMI_COL_ROWS
 #define WRFMI_COL_ROWS 1
@@ -631,18 +630,26 @@ static inline dim3 g_pt3(const Dm &d, int nk) {
   return dim3(g.x, g.y, nk);
 }
 
-// (i, j) tiles of four-point kernels covering the points from i = ibase and the rows from
-// jds - jlow through jde, nk levels: each workgroup takes 256 points of `rows` rows
-static inline dim3 g_vec(const KArgs &a, int ibase, int jlow, int rows, int nk) {
-  const Dm &d = a.d;
-  const int w = kVecTileI;
-  return dim3((d.ide - ibase + w) / w, (d.jde - d.jds + 1 + jlow + rows - 1) / rows, nk);
+// a four-point kernel over nk levels, the points from i = ibase (a multiple of four from ims)
+// through ide and the rows j0 through j1, one lane per group of four points (vec_ij)
+static void launch_vec(Launcher &L, int kid, KRef kern, int ibase, int j0, int j1, int nk) {
+  KArgs a = L.a;
+  const unsigned g = (unsigned)(a.d.ide - ibase) / kVecW + 1;
+  unsigned rows = (unsigned)L.sh[kid].rows;
+  const auto waves = [&] { return (g * (((unsigned)(j1 - j0) + rows) / rows) + 63) / 64; };
+  // waves of one workgroup share a CU's load path: with fewer workgroups than CUs (256) they are
+  // dealt out singly (48x40x20: k_tend_t_x4 17.5 us with 63 workgroups of four waves, 12 with
+  // 189 of one).  A batched launch keeps one shape for all members.
+  while (!L.rec && rows > 1 && waves() * (unsigned)nk < 256) rows /= 2;
+  a.vg = (int)g;
+  a.vmagic = g == 1 ? ~0u : (unsigned)((1ULL << 32) / g);
+  a.vi0 = ibase;
+  a.vj0 = j0;
+  L.launchK(kid, kern, dim3(waves(), 1, nk), dim3(64, rows, 1), a);
 }
-static inline dim3 g_vec3(const KArgs &a, int nk) {
-  return g_vec(a, a.d.ims + 4 * ((a.d.ids - a.d.ims) >> 2), 0, WRFMI_VEC_ROWS, nk);
+static inline void launch_vec(Launcher &L, int kid, KRef kern, int nk) {
+  launch_vec(L, kid, kern, vec_ia0(L.a.d), L.a.d.jds, L.a.d.jde, nk);
 }
-static inline dim3 vblk(const Launcher &L, int kid) { return dim3(64, (unsigned)L.sh[kid].rows, 1); }
-static inline dim3 gvec(const Launcher &L, int kid, int nk) { return g_vec(L.a, vec_ia0(L.a.d), 0, L.sh[kid].rows, nk); }
 
 // whether species m takes boundary arrays (solve_em.F:2261-2262, 2808-2810)
 static bool species_bcs(const wrfmi_config &c, const wrfmi_state &s, int m) {
@@ -656,9 +663,7 @@ static void ph_step_prep(Launcher &L) {
   const dim3 gp = g_prep(a.d);
   if (L.vec) {
     // one extra group of four below ids (mut at ids-1), rows from jds-1
-    const int ia0 = a.d.ims + 4 * ((a.d.ids - a.d.ims) >> 2) - 4;
-    L.launchK(KID_STEP_PREP, KR(k_step_prep_x4), g_vec(a, ia0, 1, L.sh[KID_STEP_PREP].rows, a.d.kde - a.d.kds + 1),
-              vblk(L, KID_STEP_PREP), a);
+    launch_vec(L, KID_STEP_PREP, KR(k_step_prep_x4), vec_ia0(a.d) - 4, a.d.jds - 1, a.d.jde, a.d.kde - a.d.kds + 1);
   } else {
     L.launchK(KID_STEP_PREP, KR(k_step_prep), dim3(gp.x, gp.y, a.d.kde - a.d.kds + 1), kColBlk, a);
   }
@@ -790,10 +795,10 @@ static void ph_tendency(Launcher &L) {
   if (L.vec && (per || L.zone_ok)) {
     // four-point kernels; on a domain with an open direction they leave the boundary zone
     // to the one-point kernels' zone form
-    L.launchK(KID_TEND_U, KR(k_tend_u_x4), gvec(L, KID_TEND_U, nk), vblk(L, KID_TEND_U), a);
-    L.launchK(KID_TEND_V, KR(k_tend_v_x4), gvec(L, KID_TEND_V, nk), vblk(L, KID_TEND_V), a);
-    L.launchK(KID_TEND_W, KR(k_tend_w_x4), gvec(L, KID_TEND_W, nk), vblk(L, KID_TEND_W), a);
-    L.launchK(KID_TEND_T, KR(k_tend_t_x4), gvec(L, KID_TEND_T, nk), vblk(L, KID_TEND_T), a);
+    launch_vec(L, KID_TEND_U, KR(k_tend_u_x4), nk);
+    launch_vec(L, KID_TEND_V, KR(k_tend_v_x4), nk);
+    launch_vec(L, KID_TEND_W, KR(k_tend_w_x4), nk);
+    launch_vec(L, KID_TEND_T, KR(k_tend_t_x4), nk);
     if (!per) {
       const dim3 gz = g_zone(a, nk);  // one level per thread
       L.launchK(KID_TEND_U, KRZ(k_tend_u), gz, kColBlk, a);
@@ -815,8 +820,8 @@ static void ph_small_prep(Launcher &L) {
   const wrfmi_state &s = a.s;
   const int nk = a.d.kde - a.d.kds + 1;
   if (L.vec) {
-    L.launchK(KID_SMALL_PREP, KR(k_small_prep_x4), gvec(L, KID_SMALL_PREP, nk), vblk(L, KID_SMALL_PREP), a);
-    L.launchK(KID_P_RHO0, KR(k_p_rho0_x4), gvec(L, KID_P_RHO0, nk - 1), vblk(L, KID_P_RHO0), a);
+    launch_vec(L, KID_SMALL_PREP, KR(k_small_prep_x4), nk);
+    launch_vec(L, KID_P_RHO0, KR(k_p_rho0_x4), nk - 1);
   } else {
     L.launchK(KID_SMALL_PREP, KR(k_small_prep), g_pt3(a.d, nk), kColBlk, a);
     L.launchK(KID_P_RHO0, KR(k_p_rho0), g_pt3(a.d, nk - 1), kColBlk, a);
@@ -845,7 +850,7 @@ static void ph_advance_uv(Launcher &L) {
     const KRef k = ks == 2 ? (per ? KRC(k_advance_uv_x4, true, 2) : KRC(k_advance_uv_x4, false, 2))
                    : ks == 8 ? (per ? KRC(k_advance_uv_x4, true, 8) : KRC(k_advance_uv_x4, false, 8))
                              : (per ? KRC(k_advance_uv_x4, true, 4) : KRC(k_advance_uv_x4, false, 4));
-    L.launchK(KID_ADVANCE_UV, k, gvec(L, KID_ADVANCE_UV, nkv), vblk(L, KID_ADVANCE_UV), L.a);
+    launch_vec(L, KID_ADVANCE_UV, k, nkv);
   } else
     L.launchK(KID_ADVANCE_UV, per ? KRP(k_advance_uv, true) : KRP(k_advance_uv, false), g_pt3(L.a.d, nkb), kColBlk, L.a);
   if (L.lbc_on) {  // spec_bdyupdate of u and v (solve_em.F:1343-1365)
@@ -863,12 +868,12 @@ static void ac_routines(Launcher &L) {
   if (L.vec) {
     const int ks = L.sh[KID_AC_DIV].levels;
     const KRef k = ks == 2 ? KRP(k_ac_div_x4, 2) : ks == 8 ? KRP(k_ac_div_x4, 8) : KRP(k_ac_div_x4, 4);
-    L.launchK(KID_AC_DIV, k, gvec(L, KID_AC_DIV, (nk + ks - 1) / ks), vblk(L, KID_AC_DIV), a);
+    launch_vec(L, KID_AC_DIV, k, (nk + ks - 1) / ks);
   }
   else L.launchK(KID_AC_DIV, KR(k_ac_div), g_pt3(a.d, nk), kColBlk, a);
   if (p64) L.launchK(KID_AC_MU_WW, KRP(k_ac_mu_ww, true), gcol(L, KID_AC_MU_WW), cblk(L, KID_AC_MU_WW), a);
   else L.launchK(KID_AC_MU_WW, KRP(k_ac_mu_ww, false), gcol(L, KID_AC_MU_WW), cblk(L, KID_AC_MU_WW), a);
-  if (L.vec) L.launchK(KID_AC_THETA, KR(k_ac_theta_x4), gvec(L, KID_AC_THETA, nk), vblk(L, KID_AC_THETA), a);
+  if (L.vec) launch_vec(L, KID_AC_THETA, KR(k_ac_theta_x4), nk);
   else L.launchK(KID_AC_THETA, KR(k_ac_theta), g_pt3(a.d, nk), kColBlk, a);
   const int pf = L.sh[KID_AC_WSOLVE].prefetch;
   KRef k;
@@ -919,8 +924,7 @@ static void ph_small_finish(Launcher &L) {
   const KArgs &a = L.a;
   const wrfmi_state &s = a.s;
   if (L.vec)
-    L.launchK(KID_SMALL_FINISH, KR(k_small_finish_x4), gvec(L, KID_SMALL_FINISH, a.d.kde - a.d.kds + 1),
-              vblk(L, KID_SMALL_FINISH), a);
+    launch_vec(L, KID_SMALL_FINISH, KR(k_small_finish_x4), a.d.kde - a.d.kds + 1);
   else L.launchK(KID_SMALL_FINISH, KR(k_small_finish), g_pt3(a.d, a.d.kde - a.d.kds + 1), kColBlk, a);
   if (a.rk_step == 3) {
     L.halo_begin();
@@ -965,8 +969,8 @@ static void ph_scalar_tend_pd(Launcher &L) {
   const Dm &d = L.a.d;
   if (L.vec && L.a.c.periodic_x && L.a.c.periodic_y) {
     const int nks = (d.kde - d.kds + kPdVK - 1) / kPdVK, nkt = (d.kde - d.kds + 1 + kPdVK - 1) / kPdVK;
-    L.launchK(KID_PD_SCALE, KR(k_pd_scale_x4), g_vec(L.a, vec_ia0(d), -1, WRFMI_VEC_ROWS, nks), kVecBlk, L.a);
-    L.launchK(KID_PD_TEND, KR(k_pd_tend_x4), g_vec(L.a, vec_ia0(d), 0, WRFMI_VEC_ROWS, nkt), kVecBlk, L.a);
+    launch_vec(L, KID_PD_SCALE, KR(k_pd_scale_x4), vec_ia0(d), d.jds, d.jde - 1, nks);
+    launch_vec(L, KID_PD_TEND, KR(k_pd_tend_x4), nkt);
     return;
   }
   const int nkz = (d.kde - d.kds + kPdK - 1) / kPdK;
@@ -988,9 +992,7 @@ static void ph_scalar_tend(Launcher &L) {
   const dim3 ga((d.ide - d.ids + 1 + kAdvTileI - 1) / kAdvTileI, (d.jde - d.jds + 1 + kAdvRows - 1) / kAdvRows,
                 (d.kde - d.kds + 1 + kAdvK - 1) / kAdvK);
   if (L.vec && (per || L.zone_ok)) {
-    const int ia0 = d.ims + 4 * ((d.ids - d.ims) >> 2);
-    const dim3 gv = g_vec(L.a, ia0, 0, L.sh[KID_ADV_SCALAR].rows, (d.kde - d.kds + kAdvVK) / kAdvVK);
-    L.launchK(KID_ADV_SCALAR, KR(k_adv_scalar_x4), gv, vblk(L, KID_ADV_SCALAR), L.a);
+    launch_vec(L, KID_ADV_SCALAR, KR(k_adv_scalar_x4), (d.kde - d.kds + kAdvVK) / kAdvVK);
     if (!per) L.launchK(KID_ADV_SCALAR, KRZ(k_adv_scalar), g_zone(L.a, d.kde - d.kds + 1), dim3(64, kAdvRows, 1), L.a);
   } else {
     L.launchK(KID_ADV_SCALAR, per ? KRP(k_adv_scalar, true) : KRP(k_adv_scalar, false), ga, dim3(64, kAdvRows, 1), L.a);
@@ -1006,8 +1008,7 @@ static void ph_scalar(Launcher &L) {
     lbc_launch(L, LBC_SPEC_TEND, 0.f, 0, L.a.c.spec_zone, {lbc_job('q', s.q_tend[m], nullptr, nullptr, nullptr, L.lbc.q_bt[m])});
   }
   if (L.vec)
-    L.launchK(KID_UPDATE_SCALAR, KR(k_update_scalar_x4), gvec(L, KID_UPDATE_SCALAR, L.a.d.kde - L.a.d.kds),
-              vblk(L, KID_UPDATE_SCALAR), L.a);
+    launch_vec(L, KID_UPDATE_SCALAR, KR(k_update_scalar_x4), L.a.d.kde - L.a.d.kds);
   else L.launchK(KID_UPDATE_SCALAR, KR(k_update_scalar), g_pt3(L.a.d, L.a.d.kde - L.a.d.kds), kColBlk, L.a);
   // flow_dep_bdy of a species without boundary arrays (solve_em.F:2342-2355, 2886-2930)
   if (L.a.c.specified && !bcs) lbc_launch(L, LBC_FLOW_DEP, 0.f, 0, L.a.c.spec_zone, {lbc_job('q', s.q[m])});
@@ -1016,17 +1017,16 @@ static void ph_scalar(Launcher &L) {
 // over species does not change any value)
 static void ph_scalar_all(Launcher &L) {
   const Dm &d = L.a.d;
-  L.launchK(KID_ADV_SCALAR, KR(k_adv_scalar_all_x4), gvec(L, KID_ADV_SCALAR, d.kde - d.kds + 1), vblk(L, KID_ADV_SCALAR), L.a);
+  launch_vec(L, KID_ADV_SCALAR, KR(k_adv_scalar_all_x4), d.kde - d.kds + 1);
   for (int m = 0; m < L.a.s.n_species; m++) {
     L.a.species = m;
     ph_scalar_mixing(L);
   }
-  L.launchK(KID_UPDATE_SCALAR, KR(k_update_scalar_all_x4), gvec(L, KID_UPDATE_SCALAR, d.kde - d.kds),
-            vblk(L, KID_UPDATE_SCALAR), L.a);
+  launch_vec(L, KID_UPDATE_SCALAR, KR(k_update_scalar_all_x4), d.kde - d.kds);
 }
 static void ph_p_rho_phi(Launcher &L) {
   if (L.vec)
-    L.launchK(KID_P_RHO_PHI, KR(k_p_rho_phi_x4), gvec(L, KID_P_RHO_PHI, L.a.d.kde - L.a.d.kds), vblk(L, KID_P_RHO_PHI), L.a);
+    launch_vec(L, KID_P_RHO_PHI, KR(k_p_rho_phi_x4), L.a.d.kde - L.a.d.kds);
   else L.launchK(KID_P_RHO_PHI, KR(k_p_rho_phi), g_pt3(L.a.d, L.a.d.kde - L.a.d.kds), kColBlk, L.a);
 }
 static void ph_bc_dry_2(Launcher &L, int kind) {
