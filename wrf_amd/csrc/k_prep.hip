@@ -1,6 +1,6 @@
 // rk_step_prep on the GPU.
 //   k_step_prep : every point-wise part, one thread per (i,k,j) point
-//   k_ww_scan   : calc_ww_cp's column sum and upward scan, one thread per (i,j) column
+//   k_ww_scan   : calc_ww_cp's column sum and upward scan, tiles of columns in LDS
 //   calculate_full   dyn_em/module_big_step_utilities_em.F:3587-3636
 //   calc_mu_uv       dyn_em/module_big_step_utilities_em.F:26-180
 //   couple_momentum  dyn_em/module_big_step_utilities_em.F:329-399
@@ -241,56 +241,96 @@ __global__ void __launch_bounds__(256) k_step_prep_x4(ARGS args) {
 }
 
 // calc_ww_cp (module_big_step_utilities_em.F:640-782): column divergence of the coupled
-// horizontal momentum and the upward scan for omega; one thread per (i, j) column.
+// horizontal momentum, its sum over the levels and the upward scan for omega.  A workgroup
+// takes kWwCols columns of the sequence of columns jds..jde-1 x ids..ide (tiles are full
+// whatever the row's width): all its threads evaluate the levels' divergence into LDS, one
+// lane per column sums and scans, so that only the sum and the scan are serial in k.  What
+// bounds it: the reads of u and v on large domains, the launch and the two serial passes on
+// small ones.  A thread that marched its column waited on 2 nz dependent loads; that against
+// this: 41x41x40 28.9 and 8.5 us, 160x128x80 69.6 and 13.9, 131x119x137 113.7 and 17.8,
+// 400x400x80 105 and 63 (2.5 TB/s), the 64-member ensemble 405 and 369.
+constexpr int kWwLevels = 160;  // levels of a column held in LDS
 template <typename ARGS, bool COMP>
-__global__ void __launch_bounds__(256) k_ww_scan(ARGS args) {
+__global__ void __launch_bounds__(kWwCols * kWwRows) k_ww_scan(ARGS args) {
+  __shared__ float divv[kWwLevels][kWwCols];
+  __shared__ float lc[kWwLevels];
   Tile3 T;
   const KArgs &a = kargs(args, T);
   const Dm &d = a.d;
   const DState &s = dstate(a);
-  const int i = col_ia(d, !std::is_same<ARGS, KArgs>::value) + (int)(T.bx * blockDim.x + threadIdx.x);
-  const int j = d.jds + (int)(T.by * blockDim.y + threadIdx.y);
-  const int ide = d.ide, jde = d.jde, kde = d.kde;
-  if (i < d.ids || i > ide || j > jde) return;
-  const bool mi = i <= ide - 1, mj = j <= jde - 1;
-  const FPtr<float> mu = s.mu_2, mub = s.mub;
-  const CPtr<float> c1h = s.c1h, c2h = s.c2h;
-  const int ktf = kde - 1;
-  // ww(1) = ww(kte) = 0 on i = its..ite
-  if (mj) {
-    s.ww[X3(d, i, 1, j)] = 0.f;
-    s.ww[X3(d, i, kde, j)] = 0.f;
+  const int col = (int)threadIdx.x, row = (int)threadIdx.y;
+  // the lane's column (vg columns per row, vmagic = 2^32 / vg: the quotient one too small at most)
+  const unsigned n = (unsigned)T.bx * kWwCols + (unsigned)col;
+  unsigned q = __umulhi(n, a.vmagic), r = n - q * (unsigned)a.vg;
+  if (r >= (unsigned)a.vg) {
+    q++;
+    r -= (unsigned)a.vg;
   }
-  if (!(mi && mj)) return;
-  // full column mass at the u points i, i+1 and v points j, j+1 (calc_ww_cp's own muu/muv)
-  const float lmuu0 = 0.5f * (((mu[X2(d, i, j)] + mub[X2(d, i, j)]) + mu[X2(d, i - 1, j)]) + mub[X2(d, i - 1, j)]);
-  const float lmuu1 = 0.5f * (((mu[X2(d, i + 1, j)] + mub[X2(d, i + 1, j)]) + mu[X2(d, i, j)]) + mub[X2(d, i, j)]);
-  const float lmuv0 = 0.5f * (((mu[X2(d, i, j)] + mub[X2(d, i, j)]) + mu[X2(d, i, j - 1)]) + mub[X2(d, i, j - 1)]);
-  const float lmuv1 = 0.5f * (((mu[X2(d, i, j + 1)] + mub[X2(d, i, j + 1)]) + mu[X2(d, i, j)]) + mub[X2(d, i, j)]);
-  const float msfuy0 = s.msfuy[X2(d, i, j)], msfuy1 = s.msfuy[X2(d, i + 1, j)];
-  const float mvi0 = s.msfvx_inv[X2(d, i, j)], mvi1 = s.msfvx_inv[X2(d, i, j + 1)];
-  const float msftx = s.msftx[X2(d, i, j)];
+  const int i = d.ids + (int)r, j = d.jds + (int)q;
+  const int kde = d.kde, ktf = kde - 1, ni = d.ni, sj = d.sj;
+  const bool in = j <= d.jde - 1, mass = in && i <= d.ide - 1;
+  const Off ob = X3(d, i, 0, j);  // level k at ob + k*ni
+  // ww(1) = ww(kte) = 0 on i = its..ite
+  if (in && row == 0) {
+    s.ww[ob + ni] = 0.f;
+    s.ww[ob + kde * ni] = 0.f;
+  }
+  float lmuu0 = 0.f, lmuu1 = 0.f, lmuv0 = 0.f, lmuv1 = 0.f, msfuy0 = 1.f, msfuy1 = 1.f, mvi0 = 1.f, mvi1 = 1.f, msftx = 1.f;
+  if (mass) {
+    // full column mass at the u points i, i+1 and v points j, j+1 (calc_ww_cp's own muu/muv)
+    const FPtr<float> mu = s.mu_2, mub = s.mub;
+    const Off o2 = X2(d, i, j);
+    lmuu0 = 0.5f * (((mu[o2] + mub[o2]) + mu[o2 - 1]) + mub[o2 - 1]);
+    lmuu1 = 0.5f * (((mu[o2 + 1] + mub[o2 + 1]) + mu[o2]) + mub[o2]);
+    lmuv0 = 0.5f * (((mu[o2] + mub[o2]) + mu[o2 - ni]) + mub[o2 - ni]);
+    lmuv1 = 0.5f * (((mu[o2 + ni] + mub[o2 + ni]) + mu[o2]) + mub[o2]);
+    msfuy0 = s.msfuy[o2];
+    msfuy1 = s.msfuy[o2 + 1];
+    mvi0 = s.msfvx_inv[o2];
+    mvi1 = s.msfvx_inv[o2 + ni];
+    msftx = s.msftx[o2];
+  }
   const float rdx = s.rdx, rdy = s.rdy;
-  float dmdt = 0.f, comp = 0.f;
-  // pass 1: divv(k) and its column sum; divv(k) is parked in ww(k+1) until the scan reads it
-  for (int k = 1; k <= ktf; k++) {
-    const Off o = X3(d, i, k, j);
-    const float c1 = c1h[X1(d, k)], c2 = c2h[X1(d, k)];
-    const float tx = (c1 * lmuu1 + c2) * s.u_2[o + 1] / msfuy1 - (c1 * lmuu0 + c2) * s.u_2[o] / msfuy0;
-    const float ty = (c1 * lmuv1 + c2) * s.v_2[o + d.sj] * mvi1 - (c1 * lmuv0 + c2) * s.v_2[o] * mvi0;
-    const float divv = msftx * s.dnw[X1(d, k)] * (rdx * tx + rdy * ty);
-    if (COMP) two_sum_acc(dmdt, comp, divv);
-    else dmdt = dmdt + divv;
-    if (k <= ktf - 1) s.ww[o + d.ni] = divv;
+  // the divergence of levels ka..kb into LDS, level k in row k - ka
+  auto levels = [&](int ka, int kb) {
+    if (mass)
+      for (int k = ka + row; k <= kb; k += kWwRows) {
+        const Off o = ob + k * ni;
+        const float c1 = s.c1h[X1(d, k)], c2 = s.c2h[X1(d, k)];
+        const float tx = (c1 * lmuu1 + c2) * s.u_2[o + 1] / msfuy1 - (c1 * lmuu0 + c2) * s.u_2[o] / msfuy0;
+        const float ty = (c1 * lmuv1 + c2) * s.v_2[o + sj] * mvi1 - (c1 * lmuv0 + c2) * s.v_2[o] * mvi0;
+        divv[k - ka][col] = msftx * s.dnw[X1(d, k)] * (rdx * tx + rdy * ty);
+      }
+    for (int k = ka + row * kWwCols + col; k <= kb; k += kWwRows * kWwCols) lc[k - ka] = s.dnw[X1(d, k)] * s.c1h[X1(d, k)];
+    __syncthreads();
+  };
+  const bool serial = mass && row == 0;
+  // columns of more than kWwLevels levels go through LDS in pieces, twice
+  float dmdt = 0.f, comp = 0.f, prev = 0.f;
+  for (int ka = 1; ka <= ktf; ka += kWwLevels) {
+    const int kb = imin(ka + kWwLevels - 1, ktf);
+    if (ka > 1) __syncthreads();
+    levels(ka, kb);
+    if (serial)
+#pragma unroll 8
+      for (int k = ka; k <= kb; k++) {
+        if (COMP) two_sum_acc(dmdt, comp, divv[k - ka][col]);
+        else dmdt = dmdt + divv[k - ka][col];
+      }
   }
   if (COMP) dmdt = dmdt + comp;
-  float prev = 0.f;
-  for (int k = 2; k <= ktf; k++) {
-    const Off o = X3(d, i, k, j);
-    const float dv = s.ww[o];
-    const float cur = prev - s.dnw[X1(d, k - 1)] * c1h[X1(d, k - 1)] * dmdt - dv;
-    s.ww[o] = cur;
-    prev = cur;
+  for (int ka = 1; ka <= ktf; ka += kWwLevels) {
+    const int kb = imin(ka + kWwLevels - 1, ktf);
+    if (ktf > kWwLevels) {
+      __syncthreads();
+      levels(ka, kb);
+    }
+    if (serial)
+#pragma unroll 8
+      for (int k = ka; k <= imin(kb, ktf - 1); k++) {  // ww(k+1) from level k
+        prev = prev - lc[k - ka] * dmdt - divv[k - ka][col];
+        s.ww[ob + (k + 1) * ni] = prev;
+      }
   }
 }
 

@@ -8,6 +8,8 @@ constexpr int kAdvK = 8;     // levels per block in k_adv_scalar
 constexpr int kTendK = 8;    // levels per thread in k_tend_u/v/w/t
 constexpr int kAdvTileI = 63;  // i points per wave in k_adv_scalar (lane 63 supplies a face)
 constexpr int kAdvRows = 4;    // j rows (waves) per block in k_adv_scalar
+// k_ww_scan's workgroup: columns (128 bytes of a level), and threads that share a column's levels
+constexpr int kWwCols = 32, kWwRows = 16;
 constexpr int kVecW = 4;       // i points per lane in the vector kernels (16-byte accesses)
 constexpr int kAdvVK = 4;      // levels per thread in k_adv_scalar_x4
 constexpr int kHaloK = 8;      // levels per thread in k_halo

@@ -667,8 +667,14 @@ static void ph_step_prep(Launcher &L) {
   } else {
     L.launchK(KID_STEP_PREP, KR(k_step_prep), dim3(gp.x, gp.y, a.d.kde - a.d.kds + 1), kColBlk, a);
   }
-  if (a.c.precision_mode == 1) L.launchK(KID_WW_SCAN, KRP(k_ww_scan, true), gcol(L, KID_WW_SCAN), cblk(L, KID_WW_SCAN), a);
-  else L.launchK(KID_WW_SCAN, KRP(k_ww_scan, false), gcol(L, KID_WW_SCAN), cblk(L, KID_WW_SCAN), a);
+  {
+    KArgs w = L.a;
+    const unsigned g = (unsigned)(a.d.ide - a.d.ids + 1), n = g * (unsigned)(a.d.jde - a.d.jds);
+    w.vg = (int)g;
+    w.vmagic = (unsigned)((1ULL << 32) / g);
+    L.launchK(KID_WW_SCAN, a.c.precision_mode == 1 ? KRP(k_ww_scan, true) : KRP(k_ww_scan, false),
+              dim3((n + kWwCols - 1) / kWwCols, 1, 1), dim3(kWwCols, kWwRows, 1), w);
+  }
   L.halo_begin();
   L.halo_add(s.ru, 'u', 1); L.halo_add(s.rv, 'v', 1); L.halo_add(s.rw, 'w', 1); L.halo_add(s.ww, 'w', 1);
   L.halo_add(s.php, 'w', 1); L.halo_add(s.alt, 't', 1); L.halo_add(s.p, 'p', 1);
