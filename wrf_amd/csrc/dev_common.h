@@ -340,6 +340,28 @@ DEVI bool point_ij(const KArgs &a, const Tile3 &T, int &i, int &j) {
   const unsigned n = ((unsigned)T.bx * blockDim.y + threadIdx.y) * blockDim.x + threadIdx.x;
   return zone_point(a.d, a.c.periodic_x, a.c.periodic_y, n, i, j);
 }
+// The launch's arguments, to be read again by every phase of a kernel: the pointers of all
+// phases together are more than the scalar registers hold, and the compiler would park them
+// in vector lanes (a readlane per use) instead of loading them again.
+DEVI const KArgs *karg_ptr(const KArgs &a) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return (const KArgs *)(const WRFMI_CONST_AS KArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+#else
+  return &a;
+#endif
+}
+DEVI const KArgs *karg_ptr(const BatchArgs &b) {
+  return (const KArgs *)(b.m + b.lut[xcd_logical(blockIdx.x, b.total)]);
+}
+DEVI const KArgs &again(const KArgs *p) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const WRFMI_CONST_AS KArgs *q = (const WRFMI_CONST_AS KArgs *)p;
+  asm volatile("" : "+s"(q));
+  return *(const KArgs *)q;
+#else
+  return *p;
+#endif
+}
 // neighbours in i of point n from the lane's group c and the groups l (i0-4..) and r (i0+4..)
 DEVI float xm1(const F4 &l, const F4 &c, int n) { return n ? c.v[n - 1] : l.v[3]; }
 DEVI float xp1(const F4 &c, const F4 &r, int n) { return n < 3 ? c.v[n + 1] : r.v[0]; }

@@ -36,28 +36,6 @@ struct alignas(16) Row {
   CT a, b, c, w;
 };
 
-// The launch's arguments, to be read again by every phase of the kernel: the pointers of all
-// phases together are more than the scalar registers hold, and the compiler would park them
-// in vector lanes (a readlane per use) instead of loading them again.
-DEVI const KArgs *karg_ptr(const KArgs &a) {
-#ifdef __HIP_DEVICE_COMPILE__
-  return (const KArgs *)(const WRFMI_CONST_AS KArgs *)__builtin_amdgcn_kernarg_segment_ptr();
-#else
-  return &a;
-#endif
-}
-DEVI const KArgs *karg_ptr(const BatchArgs &b) {
-  return (const KArgs *)(b.m + b.lut[xcd_logical(blockIdx.x, b.total)]);
-}
-DEVI const KArgs &again(const KArgs *p) {
-#ifdef __HIP_DEVICE_COMPILE__
-  const WRFMI_CONST_AS KArgs *q = (const WRFMI_CONST_AS KArgs *)p;
-  asm volatile("" : "+s"(q));
-  return *(const KArgs *)q;
-#else
-  return *p;
-#endif
-}
 #define WRFMI_PHASE \
   const KArgs &a = again(pa); \
   const Dm &d = a.d; \

@@ -17,10 +17,8 @@
 namespace wrfmi {
 
 // ------------------------------------------------------------------------------ u
-template <typename ARGS, bool PER, bool ZONE>
-__global__ void __launch_bounds__(256) k_tend_u(ARGS args) {
-  Tile3 T;
-  const KArgs &a = kargs(args, T);
+template <bool PER, bool ZONE>
+DEVI void tend_u(const KArgs &a, const Tile3 &T) {
   const Dm &d = a.d;
   const DState &s = dstate(a);
   int i, j;
@@ -434,10 +432,8 @@ __global__ void __launch_bounds__(kTallBlk) k_tend_u_x4(ARGS args) {
 }
 
 // ------------------------------------------------------------------------------ v
-template <typename ARGS, bool PER, bool ZONE>
-__global__ void __launch_bounds__(256) k_tend_v(ARGS args) {
-  Tile3 T;
-  const KArgs &a = kargs(args, T);
+template <bool PER, bool ZONE>
+DEVI void tend_v(const KArgs &a, const Tile3 &T) {
   const Dm &d = a.d;
   const DState &s = dstate(a);
   int i, j;
@@ -827,10 +823,8 @@ __global__ void __launch_bounds__(kTallBlk) k_tend_v_x4(ARGS args) {
 }
 
 // ------------------------------------------------------------------------------ w
-template <typename ARGS, bool PER, bool ZONE>
-__global__ void __launch_bounds__(256) k_tend_w(ARGS args) {
-  Tile3 T;
-  const KArgs &a = kargs(args, T);
+template <bool PER, bool ZONE>
+DEVI void tend_w(const KArgs &a, const Tile3 &T) {
   const Dm &d = a.d;
   const DState &s = dstate(a);
   int i, j;
@@ -1223,10 +1217,8 @@ __global__ void __launch_bounds__(kTallBlk) k_tend_w_x4(ARGS args) {
 }
 
 // ------------------------------------------------------------------------------ t, ph, zeroing
-template <typename ARGS, bool PER, bool ZONE>
-__global__ void __launch_bounds__(256) k_tend_t(ARGS args) {
-  Tile3 T;
-  const KArgs &a = kargs(args, T);
+template <bool PER, bool ZONE>
+DEVI void tend_t(const KArgs &a, const Tile3 &T) {
   const Dm &d = a.d;
   const DState &s = dstate(a);
   int i, j;
@@ -1686,21 +1678,60 @@ __global__ void __launch_bounds__(kTallBlk) k_tend_t_x4(ARGS args) {
   st4m(s.ph_tend, o, pt, i0, zlo(a, ids), zhi(a, ide));
 }
 
-WRFMI_INST_P2(k_tend_u, false, false)
-WRFMI_INST_P2(k_tend_u, true, false)
-WRFMI_INST_P2(k_tend_u, false, true)
+template <typename ARGS, bool PER>
+__global__ void __launch_bounds__(256) k_tend_u(ARGS args) {
+  Tile3 T;
+  const KArgs &a = kargs(args, T);
+  tend_u<PER, false>(a, T);
+}
+template <typename ARGS, bool PER>
+__global__ void __launch_bounds__(256) k_tend_v(ARGS args) {
+  Tile3 T;
+  const KArgs &a = kargs(args, T);
+  tend_v<PER, false>(a, T);
+}
+template <typename ARGS, bool PER>
+__global__ void __launch_bounds__(256) k_tend_w(ARGS args) {
+  Tile3 T;
+  const KArgs &a = kargs(args, T);
+  tend_w<PER, false>(a, T);
+}
+template <typename ARGS, bool PER>
+__global__ void __launch_bounds__(256) k_tend_t(ARGS args) {
+  Tile3 T;
+  const KArgs &a = kargs(args, T);
+  tend_t<PER, false>(a, T);
+}
+// The boundary zone (tend_* over zone_point) of all four tendencies in one launch, one after
+// the other in the level index.  They are independent, and each alone is a few workgroups
+// whose time is their latency: 4 launches of 11 to 14 us against one of 23 at 41x41x40 (the
+// step 802 and 711 us; at 200x150x50 with specified boundaries 2544 and 2488; the 64-member
+// ensemble 98.6 and 97.4 ms).
+template <typename ARGS>
+__global__ void __launch_bounds__(256) k_tend_zone(ARGS args) {
+  const KArgs *const pa = karg_ptr(args);
+  Tile3 T;
+  (void)kargs(args, T);
+  const int nk = pa->d.kde - pa->d.kds + 1, which = T.bz / nk;
+  T.bz -= which * nk;
+  if (which == 0) tend_u<false, true>(again(pa), T);
+  else if (which == 1) tend_v<false, true>(again(pa), T);
+  else if (which == 2) tend_w<false, true>(again(pa), T);
+  else tend_t<false, true>(again(pa), T);
+}
+
+WRFMI_INST(k_tend_zone)
+WRFMI_INST_P(k_tend_u, false)
+WRFMI_INST_P(k_tend_u, true)
 WRFMI_INST(k_tend_u_x4)
-WRFMI_INST_P2(k_tend_v, false, false)
-WRFMI_INST_P2(k_tend_v, true, false)
-WRFMI_INST_P2(k_tend_v, false, true)
+WRFMI_INST_P(k_tend_v, false)
+WRFMI_INST_P(k_tend_v, true)
 WRFMI_INST(k_tend_v_x4)
-WRFMI_INST_P2(k_tend_w, false, false)
-WRFMI_INST_P2(k_tend_w, true, false)
-WRFMI_INST_P2(k_tend_w, false, true)
+WRFMI_INST_P(k_tend_w, false)
+WRFMI_INST_P(k_tend_w, true)
 WRFMI_INST(k_tend_w_x4)
-WRFMI_INST_P2(k_tend_t, false, false)
-WRFMI_INST_P2(k_tend_t, true, false)
-WRFMI_INST_P2(k_tend_t, false, true)
+WRFMI_INST_P(k_tend_t, false)
+WRFMI_INST_P(k_tend_t, true)
 WRFMI_INST(k_tend_t_x4)
 
 }  // namespace wrfmi

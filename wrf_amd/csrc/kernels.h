@@ -61,18 +61,20 @@ enum Routine : int {
 };
 // Every state kernel is a template on its argument type: KArgs for one domain, BatchArgs
 // for an ensemble launch over the tiles of all members (k_halo: HaloArgs / BatchHalo).
-// ZONE = true is the one-point kernel's form over the boundary zone of a domain with an
-// open direction (zone_point), launched after the four-point form.
+// k_tend_zone, and k_adv_scalar with ZONE = true, are the one-point kernels' form over the
+// boundary zone of a domain with an open direction (zone_point), launched after the four-point
+// forms.
 template <typename A> __global__ void k_step_prep(A);
 template <typename A> __global__ void k_step_prep_x4(A);
 template <typename A, bool COMP> __global__ void k_ww_scan(A);
-template <typename A, bool PER, bool ZONE = false> __global__ void k_tend_u(A);
+template <typename A, bool PER> __global__ void k_tend_u(A);
 template <typename A> __global__ void k_tend_u_x4(A);
-template <typename A, bool PER, bool ZONE = false> __global__ void k_tend_v(A);
+template <typename A, bool PER> __global__ void k_tend_v(A);
 template <typename A> __global__ void k_tend_v_x4(A);
-template <typename A, bool PER, bool ZONE = false> __global__ void k_tend_w(A);
+template <typename A, bool PER> __global__ void k_tend_w(A);
 template <typename A> __global__ void k_tend_w_x4(A);
-template <typename A, bool PER, bool ZONE = false> __global__ void k_tend_t(A);
+template <typename A, bool PER> __global__ void k_tend_t(A);
+template <typename A> __global__ void k_tend_zone(A);
 template <typename A> __global__ void k_tend_t_x4(A);
 template <typename A> __global__ void k_small_prep(A);
 template <typename A> __global__ void k_p_rho0(A);

@@ -357,13 +357,13 @@ enum KernelId {
   KID_STEP_PREP, KID_TEND_U, KID_TEND_V, KID_TEND_W, KID_TEND_T, KID_SMALL_PREP, KID_ADVANCE_UV,
   KID_AC_DIV, KID_SMALL_FINISH, KID_ADV_SCALAR, KID_UPDATE_SCALAR, KID_P_RHO_PHI, KID_HALO, KID_P_RHO0,
   KID_COEF_W, KID_WW_SCAN, KID_AC_MU_WW, KID_AC_THETA, KID_AC_WSOLVE, KID_W_SURFACE, KID_PD_SCALE, KID_PD_TEND,
-  KID_UPDATE_SCALAR_PD, KID_DIFF6, KID_RAYLEIGH, KID_DIFF2, KID_LBC, KID_AC_COLUMN, KID_COUNT
+  KID_UPDATE_SCALAR_PD, KID_DIFF6, KID_RAYLEIGH, KID_DIFF2, KID_LBC, KID_AC_COLUMN, KID_TEND_ZONE, KID_COUNT
 };
 static const char *kKernelNames[KID_COUNT] = {
   "k_step_prep", "k_tend_u", "k_tend_v", "k_tend_w", "k_tend_t", "k_small_prep", "k_advance_uv",
   "k_ac_div", "k_small_finish", "k_adv_scalar", "k_update_scalar", "k_p_rho_phi", "k_halo", "k_p_rho0",
   "k_coef_w", "k_ww_scan", "k_ac_mu_ww", "k_ac_theta", "k_ac_wsolve", "k_set_w_surface", "k_pd_scale", "k_pd_tend",
-  "k_update_scalar_pd", "k_diff6", "k_rayleigh", "k_diff2", "k_lbc", "k_ac_column"};
+  "k_update_scalar_pd", "k_diff6", "k_rayleigh", "k_diff2", "k_lbc", "k_ac_column", "k_tend_zone"};
 struct EvPair { int id; hipEvent_t a, b; };
 static unsigned g_timing = 0;  // bit n set: time launches of kernel n
 static std::vector<EvPair> g_ev_pending;
@@ -806,11 +806,7 @@ static void ph_tendency(Launcher &L) {
     launch_vec(L, KID_TEND_W, KR(k_tend_w_x4), nk);
     launch_vec(L, KID_TEND_T, KR(k_tend_t_x4), nk);
     if (!per) {
-      const dim3 gz = g_zone(a, nk);  // one level per thread
-      L.launchK(KID_TEND_U, KRZ(k_tend_u), gz, kColBlk, a);
-      L.launchK(KID_TEND_V, KRZ(k_tend_v), gz, kColBlk, a);
-      L.launchK(KID_TEND_W, KRZ(k_tend_w), gz, kColBlk, a);
-      L.launchK(KID_TEND_T, KRZ(k_tend_t), gz, kColBlk, a);
+      L.launchK(KID_TEND_ZONE, KR(k_tend_zone), g_zone(a, 4 * nk), kColBlk, a);  // one level per thread
     }
     if (L.lbc_on) lbc_spec_dry(L);
     return;

@@ -187,9 +187,9 @@ int advect(Adv which, const float *f, const float *f_old, float *tendency, const
     launch_tiles(per ? k_adv_scalar<KArgs, true, false> : k_adv_scalar<KArgs, false, false>, g, dim3(64, kAdvRows, 1), a, st);
   } else {
     const dim3 g = pt3(d, (nk + kTendK - 1) / kTendK);
-    void (*k)(KArgs) = which == ADV_U ? (per ? k_tend_u<KArgs, true, false> : k_tend_u<KArgs, false, false>)
-                       : which == ADV_V ? (per ? k_tend_v<KArgs, true, false> : k_tend_v<KArgs, false, false>)
-                                        : (per ? k_tend_w<KArgs, true, false> : k_tend_w<KArgs, false, false>);
+    void (*k)(KArgs) = which == ADV_U ? (per ? k_tend_u<KArgs, true> : k_tend_u<KArgs, false>)
+                       : which == ADV_V ? (per ? k_tend_v<KArgs, true> : k_tend_v<KArgs, false>)
+                                        : (per ? k_tend_w<KArgs, true> : k_tend_w<KArgs, false>);
     launch_tiles(k, g, kPtBlk, a, st);
   }
   return finish(C);
