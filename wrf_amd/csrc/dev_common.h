@@ -132,6 +132,7 @@ struct KArgs {
 };
 constexpr int kKeepWW = 1;   // omega (small_step_finish reads it after the last substep)
 constexpr int kKeepAux = 2;  // t_2save and gamma (state fields no later kernel of a step reads)
+constexpr int kFoldHalo = 4;  // k_ac_column fills the (doubly periodic) halo cells of what it writes
 
 // One field of a batched halo fill (set_physical_bc3d/2d on up to 16 fields per launch)
 struct HaloField {

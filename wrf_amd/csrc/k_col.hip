@@ -174,6 +174,24 @@ DEVI void sweep_up(Row<CT> *q, int n, CT &gam, CT &wfe) {
     }
 }
 
+// A doubly periodic domain's halo cells that k_halo copies from the mass column (i, j): st(offset
+// in i, offset in j) for each of them.  With eight points or more a column has one image per axis.
+struct Images {
+  int dx = 0, dy = 0;
+  DEVI Images(const KArgs &a, int i, int j) {
+    const Dm &d = a.d;
+    if (!(a.keep & kFoldHalo)) return;
+    dx = i <= d.ids + 3 ? d.ide - d.ids : i >= d.ide - 4 ? d.ids - d.ide : 0;
+    dy = j <= d.jds + 3 ? d.jde - d.jds : j >= d.jde - 4 ? d.jds - d.jde : 0;
+  }
+  template <typename F>
+  DEVI void each(F st) const {
+    if (dx) st(dx, 0);
+    if (dy) st(0, dy);
+    if (dx && dy) st(dx, dy);
+  }
+};
+
 template <typename ARGS, typename CT, bool COMP, int C, int TASKS>
 __global__ void __launch_bounds__(kColThreads, sizeof(CT) == 4 ? 6 : 4) k_ac_column(ARGS args) {
   const KArgs *const pa = karg_ptr(args);
@@ -358,6 +376,13 @@ __global__ void __launch_bounds__(kColThreads, sizeof(CT) == 4 ? 6 : 4) k_ac_col
     c_mu[col] = mu;
     c_muts[col] = muts;
     c_muave[col] = muave;
+    const Images im(a, i, j);
+    im.each([&](int di, int dj) {
+      const Off q = o2 + (di + dj * ni);
+      s.mu_2[q] = mu;
+      s.mudf[q] = dmdt + s_mu_tend;
+      s.muts[q] = muts;
+    });
   }
   __syncthreads();
   float mu = 0.f, muts = 1.f, muave = 0.f;
@@ -637,6 +662,7 @@ __global__ void __launch_bounds__(kColThreads, sizeof(CT) == 4 ? 6 : 4) k_ac_col
   if (act) {
     WRFMI_PHASE;
     const float smdiv = a.c.smdiv;
+    const Images im(a, i, j);
 #pragma unroll
     for (int t = 0; t < TASKS; t++) {
       const int m = kl + t * KL;
@@ -651,6 +677,13 @@ __global__ void __launch_bounds__(kColThreads, sizeof(CT) == 4 ? 6 : 4) k_ac_col
         pp = pp + smdiv * (pp - q_pm1[t]);
         s.p[o] = pp;
         s.pm1[o] = ptmp;
+        im.each([&](int di, int dj) {
+          const Off q = o + (di + dj * sj);
+          s.al[q] = al;
+          s.p[q] = pp;
+          s.ph_2[q + ni] = R[m * C + col];
+          if (m == 0) s.ph_2[q] = ph_lo;
+        });
       }
     }
   }

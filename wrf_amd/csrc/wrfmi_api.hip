@@ -429,6 +429,7 @@ struct Launcher {
   RecMember *rec = nullptr;  // set: record the launches instead of enqueueing them
   bool vec = false;          // the layout allows the four-points-per-lane kernels
   bool scal_all = false;     // species advected and updated by the all-species kernels
+  bool fold_ok = false;      // k_ac_column can fill the halo cells of what it writes
   bool zone_ok = false;      // each open direction is wide enough for a boundary zone on each side
   ColShape col{0, 0};        // tiles of k_ac_column; c == 0: its four routine kernels instead
   bool whole_step = false;   // enqueued by the whole-step driver (work arrays stay internal)
@@ -886,6 +887,7 @@ static void ac_routines(Launcher &L) {
 static void ph_advance_mu_t_w(Launcher &L) {
   KArgs &a = L.a;
   const wrfmi_state &s = a.s;
+  bool fold = false;
   if (L.col.c) {
     const bool p64 = a.c.precision_mode == 1;
     const ColShape &cs = L.col;
@@ -894,6 +896,14 @@ static void ph_advance_mu_t_w(Launcher &L) {
     // and gamma as the step's last acoustic step does; a per-routine call leaves them all
     const bool end = a.iteration == a.nsmall;
     a.keep = !L.whole_step ? kKeepWW | kKeepAux : end ? kKeepWW | (a.rk_step == 3 ? kKeepAux : 0) : 0;
+    // On a doubly periodic domain the whole step's halo fills of what the column kernel writes
+    // go with its stores: as launches of their own, ten a step, the step took 543 and 518 us at
+    // 48x40x20, 2328 and 2293 at 160x128x80, 15.87 and 15.81 ms at 400x400x80.  Not with an open
+    // edge, where the rows beside it would store four times (41x41x40: 711 and 719 us, the
+    // column kernel 20 and 25), and not in a per-routine call, whose cells beyond the mass points
+    // are the caller's.
+    fold = L.whole_step && L.fold_ok;
+    if (fold) a.keep |= kFoldHalo;
     KRef k{nullptr, nullptr};
 #define COL_IS(C, T) \
   if (cs.c == C && cs.tasks == T) k = p64 ? KRCOL(double, true, C, T) : KRCOL(float, false, C, T);
@@ -917,6 +927,7 @@ static void ph_advance_mu_t_w(Launcher &L) {
     lbc_launch(L, LBC_PH_PRHO, a.dts, 0, a.c.spec_zone, {lbc_job('t', s.ph_2)}, a.c.specified);
     if (!a.c.specified) lbc_launch(L, LBC_UPDATE, a.dts, 0, a.c.spec_zone, {lbc_job('h', s.w_2, nullptr, s.rw_tend)});
   }
+  if (fold) return;
   L.halo_begin();
   L.halo_add(s.ph_2, 'w', 1); L.halo_add(s.al, 'p', 1); L.halo_add(s.p, 'p', 1);
   L.halo_add(s.muts, 't', 0); L.halo_add(s.mu_2, 't', 0); L.halo_add(s.mudf, 't', 0);
@@ -1206,6 +1217,7 @@ static int prepare(const wrfmi_state *st_in, const wrfmi_config *cfg, const wrfm
   L.col = col_shape((long)(d.ide - d.ids) * (d.jde - d.jds), d.kde - d.kds, cfg->precision_mode == 1);
   // the all-species scalar kernels (doubly periodic, aligned layout, more than one species)
   L.scal_all = L.vec && cfg->periodic_x && cfg->periodic_y && s.n_species > 1 && (own_qt || !own_scratch);
+  L.fold_ok = cfg->periodic_x && cfg->periodic_y && d.ide - d.ids >= 8 && d.jde - d.jds >= 8;
   L.zone_ok = (cfg->periodic_x || d.ide - d.ids + 1 >= 2 * kZone + 2) && (cfg->periodic_y || d.jde - d.jds + 1 >= 2 * kZone + 2);
   // specified boundaries: the four-point kernels carry the spec-zone bounds; the boundary
   // zone's one-point kernels take the relaxation rows (added to the tendencies), so those
@@ -1466,12 +1478,14 @@ extern "C" int wrfmi_ensemble_create(int n_members, const wrfmi_state *states, c
     ncol += (long)(d.ide - d.ids) * (d.jde - d.jds);
   }
   const ColShape col = col_shape(ncol, nz_max, cfgs[0].precision_mode == 1);
-  bool all_zone = true;
+  bool all_zone = true, all_fold = true;
+  for (int m = 0; m < n_members && !rc; m++) all_fold = all_fold && Ls[m].fold_ok;
   for (int m = 0; m < n_members && !rc; m++) all_zone = all_zone && Ls[m].zone_ok;
   for (int m = 0; m < n_members && !rc; m++) {
     Ls[m].vec = all_vec;
     Ls[m].scal_all = Ls[m].scal_all && all_vec;
     Ls[m].zone_ok = all_zone;
+    Ls[m].fold_ok = all_fold;
     Ls[m].col = col;
     Ls[m].rec = &rec[m];
     enqueue_step(Ls[m]);
